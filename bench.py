@@ -242,7 +242,7 @@ def bench_gemv(gs, torch, steps=50, warmup=5, cpu=True):
     torch.cuda.synchronize()
     us = e0.elapsed_time(e1) / steps * 1e3
     nbytes = workloads.qmatrix_bytes(qt, rows, cols) + 4 * cols + 4 * rows
-    out = {"kernel": "gs::q6k_gemv_xreg", "qtype": "Q6_K", "rows": rows, "cols": cols, "B": 1,
+    out = {"kernel": "gs::qgemv_kernel", "qtype": "Q6_K", "rows": rows, "cols": cols, "B": 1,
            "us": us, "bytes_per_launch": nbytes,
            "roofline": {"bound": "hbm", "achieved": nbytes / us / 1e3, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                         "frac": nbytes / us / 1e3 / PEAK_HBM_GBS}}

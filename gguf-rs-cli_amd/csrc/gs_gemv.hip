@@ -1,29 +1,28 @@
-// gs_gemv.hip -- gfx950 quantized matrix-vector product that produces the
-// logits (the reference's output projection, src/model/llama.rs:333-334 on
-// the GPU path, :405-407 on the CPU path), for Q4_0, Q4_1, Q8_0, Q3_K, Q4_K,
-// Q5_K and Q6_K weights.
+// gs_gemv.hip -- gfx950 quantized projection that produces the logits (the
+// reference's output projection, src/model/llama.rs:333-334 on the GPU path,
+// :405-407 on the CPU path), for Q4_0, Q4_1, Q8_0, Q3_K, Q4_K, Q5_K and Q6_K
+// weights: out[b][r] = sum_c W[r][c] x[b][c] for B vectors.
 //
-// HBM-bound: every weight byte is read once per call and nothing else of
-// size moves.  Device layout (rearranged at upload from the GGUF blocks, the
-// same 210 / 34 bytes per block as the file), chosen so that every load
-// instruction of a wave reads one contiguous run of memory:
-//   Q6_K: three planes of 16-byte chunks, one chunk per quarter block and
-//         plane (ql[64h + l0 ..], ql[64h + 32 + l0 ..], qh[32h + l0 ..] for
-//         quarter (h, l0), see below), indexed row * 4nb + quarter; a plane of
-//         32-bit words, the quarter's four int8 scales; the f16 d per block.
-//   Q8_0: 16-byte chunks of int8 quants, row * 2nb + half block; f16 d per block.
-// Weight loads are non-temporal (each byte is used once).
+// Two kernels, for up to 4 vectors and for more, on the matrix cores, for
+// every type and row length.  The stored integers of a weight are exact in
+// f16 (at most 8 bits; Q3_K's scaled by its 6-bit sub-block scale: at most
+// 9), and x is split into two f16 parts, x s = hi + lo with s a power of two,
+// whose products the MFMA adds in f32.  What is left for the vector units is
+// the unpacking of the integers (about 1.3 instructions per weight for the
+// 4-bit types) and a multiply-add per sub-block, row and vector.
 //
-// One wave per row, rows strided over all waves of the grid.  A lane takes a
-// fixed slice of the columns (Q6_K: a quarter block, 64 weights = 16 values
-// of l in one half of a block; Q8_0: half blocks of 16 weights), so its slice
-// of x stays in registers for every row the wave visits (when a row fits in
-// one pass of the wave, cols <= 4096), with the sums of x over its 16-weight
-// groups.  Weights are decoded four to a 32-bit word and converted with the
-// byte-to-float instructions; the offset of the stored values (Q6_K q + 32,
-// Q8_0 q + 128 after flipping the sign bit) is taken out once per group:
-// sum (u - o) x = sum u x - o * sum x.  The next row's loads are issued
-// before the current row is computed.
+// Why: the weights have to be read once per call, and that read is the bound
+// up to about 16 vectors.  Byte-to-float conversions and FMAs took 3.2-3.4
+// instructions per weight, as long as the read itself, for one vector, and a
+// pass over the weights for each further one.  Measured (MI355X, us per call;
+// before: one pass per vector):
+//   Q4_K 152064 x 3584:  1 vector 61-68 -> 50 (6.1 TB/s), 16: 980 -> 77,
+//                        32: 1960 -> 115
+//   Q6_K 152064 x 3584:  1 vector 72.4 -> 72.6 (6.2 TB/s), 32: 2340 -> 160
+//   Q5_K 32000 x 8192:   1 vector 121 -> 38
+//   Q8_0 32000 x 4096:   4 vectors 100 -> 23
+// The error against 64-bit sums is 1.0e-7 to 2.0e-7 (2-norm, relative) where
+// it was 1.4e-7 to 2.1e-7.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>
@@ -34,927 +33,1005 @@
 
 namespace gs {
 
-constexpr int kGemvThreads = 256;       // 4 waves per workgroup
-constexpr int kMaxCols = 16384;         // x staged in LDS (64 KB) on the general path
+constexpr int kMaxCols = 16384;
+constexpr int kPair = 256;              // columns of a record (eight K steps of 32)
 
-__device__ __forceinline__ float h2f(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
 
-// Streaming loads of the weights (read once per call: non-temporal).
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint4 ntl4(const void *p)
+__device__ __forceinline__ float h2f(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
+__device__ __forceinline__ h2_t as_h2(uint32_t w) { return __builtin_bit_cast(h2_t, w); }
+__device__ __forceinline__ h2_t splat(float f) { return h2_t{(_Float16)f, (_Float16)f}; }
+__device__ __forceinline__ h8_t cat(h2_t a, h2_t b, h2_t c, h2_t d) { return h8_t{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y}; }
+__device__ __forceinline__ h4_t cat(h2_t a, h2_t b) { return h4_t{a.x, a.y, b.x, b.y}; }
+__device__ __forceinline__ float ub(uint32_t w, int t) { return (float)((w >> (8 * t)) & 0xffu); }
+
+// The records are read through an opaque scalar address in the global address
+// space: one scalar base per record and 32-bit lane offsets (a generic one
+// would make flat loads, whose waits are for everything).  Non-temporal: each
+// byte is used once, and kept out of the way of what is not (Q4_K 152064 x
+// 3584, one vector: 59 us against 62).
+#define GS_GLOBAL __attribute__((address_space(1)))
+typedef const GS_GLOBAL uint8_t *gptr;
+__device__ __forceinline__ gptr opaque(const uint8_t *p)
 {
-    const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p));
-    return make_uint4(v.x, v.y, v.z, v.w);
+    uint64_t a = (uint64_t)p;
+    asm volatile("" : "+s"(a));
+    return (gptr)a;
 }
-__device__ __forceinline__ uint2 ntl2(const void *p)
+template <class T> __device__ __forceinline__ T ld(gptr p, uint32_t off)
 {
-    const u32x2_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t *>(p));
-    return make_uint2(v.x, v.y);
+    return __builtin_nontemporal_load((const GS_GLOBAL T *)(p + off));
 }
 
-__device__ __forceinline__ float wave_sum(float v)
+// Integers in 16-bit halves to f16: 0x6400 | n is 1024 + n for n < 1024.
+// n0: n in the low bits of the halves; n4: 16 n in bits 4 and up (a nibble in
+// place, not shifted down): (1024 + 16 n) / 16 = 64 + n, exact in one fma.
+constexpr uint32_t kMagic = 0x64006400u;
+// A constant that the compiler keeps in a scalar (vector) register: with
+// literals (w & mask) | c takes two instructions, the three-operand form has
+// none.  (No instruction in the asm: the compiler does not see the hazards
+// between one and the MFMAs around it.)
+__device__ __forceinline__ uint32_t sreg(uint32_t c)
 {
+    uint32_t r;
+    asm("" : "=s"(r) : "0"(c));
+    return r;
+}
+__device__ __forceinline__ uint32_t vreg(uint32_t c)
+{
+    uint32_t r;
+    asm("" : "=v"(r) : "0"(c));
+    return r;
+}
+__device__ __forceinline__ uint32_t and_or(uint32_t w, uint32_t mask, uint32_t c)
+{
+    uint32_t d = (w & sreg(mask)) | c;
+    asm("" : "+v"(d));          // (two in a row stay two: not two ands and a three-way or)
+    return d;
+}
+__device__ __forceinline__ h2_t n0(uint32_t w, float off) { return as_h2(w) - splat(1024.0f + off); }
+__device__ __forceinline__ h2_t n4(uint32_t w, float off)
+{
+    return __builtin_elementwise_fma(as_h2(w), splat(0.0625f), splat(-64.0f - off));
+}
+__device__ __forceinline__ h2_t u0(uint32_t w, float off) { return n0(and_or(w, 0x000F000Fu, vreg(kMagic)), off); }
+__device__ __forceinline__ h2_t u4(uint32_t w, float off) { return n4(and_or(w, 0x00F000F0u, vreg(kMagic)), off); }
+
+// ------------------------------------------------------- operand layouts ---
+// v_mfma_f32_16x16x32_f16, lane L = 16 g + n: operand A holds row n, k = 8 g
+// .. 8 g + 7 (x); operand B column n, the same k (weight row n of the tile);
+// D column n, rows 4 g .. 4 g + 3.  (16x16x16: k = 4 g .. 4 g + 3.)  With the
+// weights as B, everything of a weight row (bits, scales, sums) sits in the
+// lanes with that n.
+__device__ __forceinline__ f4_t mfma(h8_t a, h8_t b, f4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f4_t mfma(h4_t a, h4_t b, f4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
+constexpr f4_t kZero = {0.0f, 0.0f, 0.0f, 0.0f};
+
+// ------------------------------------------------------------- formats -----
+// A record holds 256 columns of 16 rows, in the order the lanes read them:
+// 16-byte pieces for all 64 lanes first (lane L at 16 L), then what is per
+// row.  Records of a tile follow each other, so a wave reads one run of
+// memory.  Each format has
+//   kRec   bytes of a record;
+//   kSplit a lane's columns of K step ks: 32 ks + 4 g .. + 3 and + 16 (true)
+//          or 32 ks + 8 g .. + 7;
+//   kSwap  within four columns the unpacked order is 0, 2, 1, 3 (bytes 0 and
+//          2 of a word, then 1 and 3);
+//   kHalf  a scale for each 16 columns, and an operand for each (their first
+//          four columns of a lane, and the other four);
+//   kChain the sub-block scales are in the operands;
+//   kRecScale a factor of the whole record, rec();
+//   kMin   a term min_scale() * (min_frag() . the sums of x over 32 columns);
+//   Item, load(); frag(): the operand of a step (and half of it); sub(): its
+//          scale;
+//   put(): a lane's part of a record from the 256 (or 8 x 32) GGUF blocks of
+//          its row.
+
+// A row's blocks from a record on: b, bb bytes each, n of them left (0 bytes
+// past the row's end).
+struct Src {
+    const uint8_t *b;
+    int bb, n;
+    __device__ uint32_t at(int j, int i) const { return j < n ? b[(size_t)j * bb + i] : 0u; }
+    __device__ uint32_t word(int j, int i) const   // four bytes, no alignment
+    {
+        return at(j, i) | at(j, i + 1) << 8 | at(j, i + 2) << 16 | at(j, i + 3) << 24;
+    }
+    __device__ uint32_t half(int j, int i) const { return at(j, i) | at(j, i + 1) << 8; }
+};
+
+// Bytes 2 i, 2 i + 1 of w as integers less off.
+__device__ __forceinline__ h2_t two(uint32_t w, int i, float off)
+{
+    h2_t d = as_h2(__builtin_amdgcn_perm(kMagic, w, i ? 0x07030702u : 0x07010700u)) - splat(1024.0f + off);
+    asm("" : "+v"(d));          // (one packed subtraction, also where the halves are used apart)
+    return d;
+}
+
+// Q4_0 (src/tensor/dequant.rs:26-41) w = (q - 8) d; Q4_1 (:42-54) w = q d + m;
+// byte l of a block's 16 holds weight l (low nibble) and l + 16 (high).
+template <bool Q41> struct Q4Fmt {
+    static constexpr int kRec = 2048 + 256 + (Q41 ? 256 : 0), kBlock = Q41 ? 20 : 18, kCols = 32;
+    static constexpr bool kSplit = true, kSwap = true, kHalf = false, kChain = false, kRecScale = false, kMin = Q41;
+    struct Item { u4_t q[2], d, m; };
+    static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
+    {
+        it.q[0] = ld<u4_t>(r, 16 * lane);
+        it.q[1] = ld<u4_t>(r, 1024 + 16 * lane);
+        it.d = ld<u4_t>(r, 2048 + 16 * (lane & 15));
+        if (Q41) it.m = ld<u4_t>(r, 2304 + 16 * (lane & 15));
+    }
+    static __device__ __forceinline__ h8_t frag(const Item &it, int ks)
+    {
+        constexpr float off = Q41 ? 0.0f : 8.0f;
+        const uint32_t w = it.q[ks >> 2][ks & 3], h = w >> 8;
+        return cat(u0(w, off), u0(h, off), u4(w, off), u4(h, off));
+    }
+    static __device__ __forceinline__ float sub(const Item &it, int ks, int) { return h2f(it.d[ks >> 1] >> (16 * (ks & 1))); }
+    static __device__ __forceinline__ float rec(const Item &) { return 1.0f; }
+    static __device__ __forceinline__ h8_t min_frag(const Item &it) { return __builtin_bit_cast(h8_t, it.m); }
+    static __device__ __forceinline__ float min_scale(const Item &) { return 64.0f; }
+    static __device__ void put(uint8_t *r, const Src &s, int lane)
+    {
+        const int g = lane >> 4, n = lane & 15, o = Q41 ? 4 : 2;
+        for (int ks = 0; ks < 8; ks++)
+            reinterpret_cast<uint32_t *>(r + 1024 * (ks >> 2) + 16 * lane)[ks & 3] = s.word(ks, o + 4 * g);
+        for (int k = 0; k < 2; k++) {
+            const int ks = 2 * g + k;
+            reinterpret_cast<uint16_t *>(r + 2048 + 16 * n)[ks] = (uint16_t)s.half(ks, 0);
+            if (Q41) reinterpret_cast<uint16_t *>(r + 2304 + 16 * n)[ks] = (uint16_t)s.half(ks, 2);
+        }
+    }
+};
+
+// Q8_0: w = q d, int8 q, stored as q + 128.
+struct Q8Fmt {
+    static constexpr int kRec = 4096 + 256, kBlock = 34, kCols = 32;
+    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kChain = false, kRecScale = false, kMin = false;
+    struct Item { u4_t q[4], d; };
+    static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
+    {
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
-    return v;
+        for (int i = 0; i < 4; i++) it.q[i] = ld<u4_t>(r, 1024 * i + 16 * lane);
+        it.d = ld<u4_t>(r, 4096 + 16 * (lane & 15));
+    }
+    static __device__ __forceinline__ h8_t frag(const Item &it, int ks)
+    {
+        const uint32_t w0 = it.q[ks >> 1][2 * (ks & 1)], w1 = it.q[ks >> 1][2 * (ks & 1) + 1];
+        return cat(two(w0, 0, 128.0f), two(w0, 1, 128.0f), two(w1, 0, 128.0f), two(w1, 1, 128.0f));
+    }
+    static __device__ __forceinline__ float sub(const Item &it, int ks, int) { return h2f(it.d[ks >> 1] >> (16 * (ks & 1))); }
+    static __device__ __forceinline__ float rec(const Item &) { return 1.0f; }
+    static __device__ void put(uint8_t *r, const Src &s, int lane)
+    {
+        const int g = lane >> 4, n = lane & 15;
+        for (int ks = 0; ks < 8; ks++)
+            for (int k = 0; k < 2; k++)
+                reinterpret_cast<uint32_t *>(r + 1024 * (ks >> 1) + 16 * lane)[2 * (ks & 1) + k] =
+                    s.word(ks, 2 + 8 * g + 4 * k) ^ 0x80808080u;
+        for (int k = 0; k < 2; k++)
+            reinterpret_cast<uint16_t *>(r + 4096 + 16 * n)[2 * g + k] = (uint16_t)s.half(2 * g + k, 0);
+    }
+};
+
+// get_scale_min_k4 (src/tensor/dequant.rs:141-148): the 6-bit scale (min) of
+// sub-block j from the 12 packed bytes at `o`.
+__device__ inline uint32_t k4_scale(const Src &s, int o, int j)
+{
+    return j < 4 ? s.at(0, o + j) & 63u : (s.at(0, o + j + 4) & 15u) | (s.at(0, o + j - 4) >> 6) << 4;
+}
+__device__ inline uint32_t k4_min(const Src &s, int o, int j)
+{
+    return j < 4 ? s.at(0, o + j + 4) & 63u : s.at(0, o + j + 4) >> 4 | (s.at(0, o + j) >> 6) << 4;
 }
 
-// Row sums of kRB rows at once (kRB = 4, 8 or 16): each lane's partial of
-// row k is written to the wave's LDS tile t[k][lane]; lane L then adds the
-// 64 kRB / 64 partials t[L % kRB][..] of its share, and log2(64 / kRB)
-// shuffles combine the shares.  Lanes 0 .. kRB-1 return the sums of rows
-// 0 .. kRB-1.
-template <int kRB>
-__device__ __forceinline__ float rows_sum(float (&part)[kRB], float *t)
-{
-    const int lane = threadIdx.x & 63;
+// Q4_K / Q5_K (src/tensor/dequant.rs:149-196): w = (d sc_i) q - dmin m_i per
+// sub-block i of 32; byte 32 s + l of qs holds weight 64 s + l (low nibble,
+// i = 2 s) and 64 s + 32 + l (high, i = 2 s + 1); Q5_K adds bit i of qh[l]
+// as 16.  A lane's bits of qh for two steps s are one word: bits b, b + 16
+// (low nibbles) and b + 1, b + 17 (high), b = 8 (s & 1) + 2 q, for the bytes
+// 0 and 2 of the lane's first word (q = 0), 1 and 3 of it (1), and the
+// second word's (2, 3): one shift and mask moves a pair to the places above
+// the nibbles.
+template <bool Q5> struct KFmt {
+    static constexpr int kRec = 2048 + (Q5 ? 512 : 0) + 256 + 64, kBlock = Q5 ? 176 : 144, kCols = 256;
+    static constexpr bool kSplit = false, kSwap = true, kHalf = false, kChain = false, kRecScale = true, kMin = true;
+    struct Item { u4_t q[2]; u2_t h, sc, mn; uint32_t dd; };
+    static constexpr int kH = 2048, kS = 2048 + (Q5 ? 512 : 0), kM = kS + 128, kD = kS + 256;
+    static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
+    {
+        it.q[0] = ld<u4_t>(r, 16 * lane);
+        it.q[1] = ld<u4_t>(r, 1024 + 16 * lane);
+        if (Q5) it.h = ld<u2_t>(r, kH + 8 * lane);
+        it.sc = ld<u2_t>(r, kS + 8 * (lane & 15));
+        it.mn = ld<u2_t>(r, kM + 8 * (lane & 15));
+        it.dd = ld<uint32_t>(r, kD + 4 * (lane & 15));
+    }
+    static __device__ __forceinline__ h8_t frag(const Item &it, int ks)
+    {
+        const int st = ks >> 1;
+        const uint32_t w0 = it.q[st >> 1][2 * (st & 1)], w1 = it.q[st >> 1][2 * (st & 1) + 1];
+        const bool hi = ks & 1;
+        uint32_t w[4] = {w0, w0 >> 8, w1, w1 >> 8};
 #pragma unroll
-    for (int k = 0; k < kRB; k++) t[k * 64 + lane] = part[k];
+        for (int q = 0; q < 4; q++) {
+            w[q] = and_or(w[q], hi ? 0x00F000F0u : 0x000F000Fu, vreg(kMagic));
+            if constexpr (Q5) {
+                const uint32_t hw = it.h[st >> 1];
+                const int up = (hi ? 7 : 4) - (8 * (st & 1) + 2 * q);      // to bit 4, or 8 (from b + 1)
+                w[q] = and_or(up > 0 ? hw << up : hw >> -up, hi ? 0x01000100u : 0x00100010u, w[q]);
+            }
+        }
+        return hi ? cat(n4(w[0], 0.0f), n4(w[1], 0.0f), n4(w[2], 0.0f), n4(w[3], 0.0f))
+                  : cat(n0(w[0], 0.0f), n0(w[1], 0.0f), n0(w[2], 0.0f), n0(w[3], 0.0f));
+    }
+    static __device__ __forceinline__ float sub(const Item &it, int ks, int) { return ub(it.sc[ks >> 2], ks & 3); }
+    static __device__ __forceinline__ float rec(const Item &it) { return h2f(it.dd & 0xffffu); }
+    static __device__ __forceinline__ h8_t min_frag(const Item &it)
+    {
+        return cat(two(it.mn[0], 0, 0.0f), two(it.mn[0], 1, 0.0f), two(it.mn[1], 0, 0.0f), two(it.mn[1], 1, 0.0f));
+    }
+    static __device__ __forceinline__ float min_scale(const Item &it) { return -64.0f * h2f(it.dd >> 16); }
+    static __device__ void put(uint8_t *r, const Src &s, int lane)
+    {
+        const int g = lane >> 4, n = lane & 15, qs = Q5 ? 48 : 16;
+        for (int st = 0; st < 4; st++)
+            for (int k = 0; k < 2; k++)
+                reinterpret_cast<uint32_t *>(r + 1024 * (st >> 1) + 16 * lane)[2 * (st & 1) + k] =
+                    s.word(0, qs + 32 * st + 8 * g + 4 * k);
+        if (Q5) {
+            for (int hw = 0; hw < 2; hw++) {
+                uint32_t w = 0;
+                for (int st = 0; st < 2; st++)
+                    for (int q = 0; q < 4; q++)
+                        for (int e = 0; e < 2; e++) {
+                            const uint32_t qh = s.at(0, 16 + 8 * g + 4 * (q >> 1) + (q & 1) + 2 * e);
+                            const int i = 2 * (2 * hw + st), b = 8 * st + 2 * q + 16 * e;
+                            w |= (qh >> i & 1u) << b | (qh >> (i + 1) & 1u) << (b + 1);
+                        }
+                reinterpret_cast<uint32_t *>(r + kH + 8 * lane)[hw] = w;
+            }
+        }
+        for (int k = 0; k < 2; k++) {
+            r[kS + 8 * n + 2 * g + k] = (uint8_t)k4_scale(s, 4, 2 * g + k);
+            r[kM + 8 * n + 2 * g + k] = (uint8_t)k4_min(s, 4, 2 * g + k);
+        }
+        if (g == 0) reinterpret_cast<uint32_t *>(r + kD)[n] = s.word(0, 0);   // d | dmin << 16
+    }
+};
+
+// Q6_K (src/tensor/dequant.rs:203-214): w = (d sc) (u - 32), an int8 scale
+// per 16 weights; weight 128 h + 32 j + l takes a nibble of
+// ql[64 h + 32 (j & 1) + l] (low for j < 2) and bits 2 j of qh[32 h + l].
+// The scales' products need 12 bits, more than an f16 holds: each 16 columns
+// are summed apart and scaled in f32.
+struct Q6Fmt {
+    static constexpr int kRec = 2048 + 1024 + 256 + 32, kBlock = 210, kCols = 256;
+    static constexpr bool kSplit = true, kSwap = true, kHalf = true, kChain = false, kRecScale = true, kMin = false;
+    struct Item { u4_t q[2], c, sc; uint32_t d; };
+    static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
+    {
+        it.q[0] = ld<u4_t>(r, 16 * lane);
+        it.q[1] = ld<u4_t>(r, 1024 + 16 * lane);
+        it.c = ld<u4_t>(r, 2048 + 16 * lane);
+        it.sc = ld<u4_t>(r, 3072 + 16 * (lane & 15));
+        it.d = ld<uint16_t>(r, 3328 + 2 * (lane & 15));
+    }
+    // columns 16 i .. + 15 of step ks = 4 h + j
+    static __device__ __forceinline__ h4_t frag(const Item &it, int ks, int i)
+    {
+        const int h = ks >> 2, j = ks & 3;
+        const uint32_t a = it.q[h][2 * (j & 1) + i], c = it.c[2 * h + i], e = j & 1 ? c << 2 : c << 4, f = j & 1 ? c >> 6 : c >> 4;
+        return j < 2 ? cat(n0(and_or(e, 0x00300030u, and_or(a, 0x000F000Fu, vreg(kMagic))), 32.0f),
+                           n0(and_or(f, 0x00300030u, and_or(a >> 8, 0x000F000Fu, vreg(kMagic))), 32.0f))
+                     : cat(n4(and_or(e, 0x03000300u, and_or(a, 0x00F000F0u, vreg(kMagic))), 32.0f),
+                           n4(and_or(f, 0x03000300u, and_or(a >> 8, 0x00F000F0u, vreg(kMagic))), 32.0f));
+    }
+    // (an f16: two scales in two instructions, and the multiply-add takes it as it is)
+    static __device__ __forceinline__ float sub(const Item &it, int ks, int i) { return (float)two(it.sc[ks >> 1], ks & 1, 128.0f)[i]; }
+    static __device__ __forceinline__ float rec(const Item &it) { return h2f(it.d); }
+    static __device__ void put(uint8_t *r, const Src &s, int lane)
+    {
+        const int g = lane >> 4, n = lane & 15;
+        for (int h = 0; h < 2; h++) {
+            for (int i = 0; i < 2; i++) {
+                uint32_t *q = reinterpret_cast<uint32_t *>(r + 1024 * h + 16 * lane);
+                q[i] = s.word(0, 64 * h + 16 * i + 4 * g);
+                q[2 + i] = s.word(0, 64 * h + 32 + 16 * i + 4 * g);
+                reinterpret_cast<uint32_t *>(r + 2048 + 16 * lane)[2 * h + i] = s.word(0, 128 + 32 * h + 16 * i + 4 * g);
+            }
+        }
+        reinterpret_cast<uint32_t *>(r + 3072 + 16 * n)[g] = s.word(0, 192 + 4 * g) ^ 0x80808080u;    // scale + 128
+        if (g == 0) reinterpret_cast<uint16_t *>(r + 3328)[n] = (uint16_t)s.half(0, 208);
+    }
+};
+
+// Q3_K in the GGUF layout: w = d sc (u - 4), a signed 6-bit scale per 16
+// weights; weight 128 h + 32 j + l has low bits (qs[32 h + l] >> 2 j) & 3 and
+// third bit (hmask[l] >> (4 h + j)) & 1.  The three bits are merged into a
+// nibble here (146 bytes per block on the device for the file's 110): a
+// lane's eight weights of a step are the nibbles 0, 4, 1, 5, 2, 6, 3, 7 of
+// its word.  |sc (u - 4)| <= 128 is exact in f16, so the scale goes into the
+// weights and a record is one chain of MFMAs.
+struct Q3Fmt {
+    static constexpr int kRec = 2048 + 256 + 32, kBlock = 110, kCols = 256;
+    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kChain = true, kRecScale = true, kMin = false;
+    struct Item { u4_t q[2]; u2_t sc; uint32_t d; };
+    static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
+    {
+        it.q[0] = ld<u4_t>(r, 16 * lane);
+        it.q[1] = ld<u4_t>(r, 1024 + 16 * lane);
+        it.sc = ld<u2_t>(r, 2048 + 8 * (lane & 15) + 128 * (lane >> 5));
+        it.d = ld<uint16_t>(r, 2304 + 2 * (lane & 15));
+    }
+    static __device__ __forceinline__ h8_t frag(const Item &it, int ks)
+    {
+        const uint32_t w = it.q[ks >> 2][ks & 3], h = w >> 8, p = ks & 3;
+        const h2_t sc = as_h2(__builtin_amdgcn_perm(kMagic, it.sc[ks >> 2], 0x07000700u | p << 16 | p)) - splat(1024.0f + 32.0f);
+        return cat(u0(w, 4.0f) * sc, u4(w, 4.0f) * sc, u0(h, 4.0f) * sc,
+                   u4(h, 4.0f) * sc);
+    }
+    static __device__ __forceinline__ float sub(const Item &, int, int) { return 1.0f; }
+    static __device__ __forceinline__ float rec(const Item &it) { return h2f(it.d); }
+    // The scale of sub-block is, plus 32: low nibble from byte is % 8 (bits
+    // 0-3 for is < 8, 4-7 above), top two bits from bits 2 (is / 4) of byte
+    // 8 + is % 4.
+    static __device__ uint32_t scale(const Src &s, int is)
+    {
+        const int k = is >> 2, j = is & 3;
+        const uint32_t b = s.at(0, 96 + (k & 1) * 4 + j);
+        return (k < 2 ? b & 15u : b >> 4) | (s.at(0, 104 + j) >> (2 * k) & 3u) << 4;
+    }
+    static __device__ void put(uint8_t *r, const Src &s, int lane)
+    {
+        const int g = lane >> 4, n = lane & 15;
+        for (int ks = 0; ks < 8; ks++) {
+            const int h = ks >> 2, j = ks & 3;
+            uint32_t w = 0;
+            for (int i = 0; i < 8; i++) {
+                const int l = 8 * g + i;
+                const uint32_t u = (s.at(0, 32 + 32 * h + l) >> (2 * j) & 3u) | (s.at(0, l) >> (4 * h + j) & 1u) << 2;
+                w |= u << (4 * (i >> 1) + 16 * (i & 1));
+            }
+            reinterpret_cast<uint32_t *>(r + 1024 * h + 16 * lane)[j] = w;
+        }
+        if ((g & 1) == 0)       // lanes 16 g, 16 (g + 1) share the 16-column half g / 2 of a step
+            for (int ks = 0; ks < 8; ks++)
+                r[2048 + 8 * n + 128 * (g >> 1) + ks] = (uint8_t)scale(s, 2 * ks + (g >> 1));
+        if (g == 0) reinterpret_cast<uint16_t *>(r + 2304)[n] = (uint16_t)s.half(0, 108);
+    }
+};
+
+// ------------------------------------------------------- x in f16 parts ----
+// x s = hi + lo, s = 2^(13 - e) for the largest |x| in [2^e, 2^(e+1)) of the
+// columns that share s, and (kMin) the sums of x s over 32 columns, over 64,
+// in three parts.  The parts hold 22 bits of every x above 2^-24 of the
+// largest, and 2^-39 of the largest at worst.
+__device__ __forceinline__ void x_scale(float mx, float &s, float &inv)
+{
+    // 2^(13 - e), at most 2^126, and its inverse (exact; e of a subnormal as
+    // -127, of an infinity as 128)
+    const int e = (int)(__float_as_uint(mx) >> 23) - 127;
+    const int se = mx > 0.0f ? min(13 - e, 126) : 0;
+    s = __uint_as_float((uint32_t)(se + 127) << 23);
+    inv = __uint_as_float((uint32_t)(127 - se) << 23);
+}
+// (For an infinite t the difference is a NaN, which the clamp drops: hi
+// alone decides the sum.)
+__device__ __forceinline__ void x_split(float t, _Float16 &hi, _Float16 &lo)
+{
+    hi = (_Float16)t;
+    lo = (_Float16)__builtin_amdgcn_fmed3f(t - (float)hi, -4.0f, 4.0f);
+}
+__device__ __forceinline__ void x_split3(float t, _Float16 &a, _Float16 &b, _Float16 &c)
+{
+    a = (_Float16)t;
+    const float r = __builtin_amdgcn_fmed3f(t - (float)a, -4.0f, 4.0f);
+    b = (_Float16)r;
+    c = (_Float16)(r - (float)b);
+}
+template <class F> constexpr int x_pos(int i)   // place of column i of four
+{
+    return F::kSwap && (i == 1 || i == 2) ? 3 - i : i;
+}
+
+// ------------------------------------------------- up to 4 vectors (GEMV) ---
+// Rows 4 v, 4 v + 1 of A = hi, lo of vector v (the others zero): one MFMA per
+// step, and a lane's sum of vector g is D[0] + D[1].  Formats with a scale
+// for each 16 columns (kHalf) use all four rows: x of the first 16 columns
+// of the step in rows 4 v, 4 v + 1 (zeros for the others) and of the second
+// in 4 v + 2, 4 v + 3, so that D[2] + D[3] is the second half's sum.
+//
+// A block takes tpb tiles of 16 rows; its waves share the columns, a record
+// each, with their operands of x in registers for all tiles.  D tiles are in
+// flight: a record's registers are loaded again, for the tile D further on,
+// as soon as it has been used.  The waves' sums meet in LDS every kBatch
+// tiles (two buffers: one barrier per batch); within a batch a wave's
+// priority falls with its progress, so that the waves of a SIMD arrive
+// together (with equal priorities the youngest came late and ran the end of
+// each batch alone: Q4_K 152064 x 3584 59 us against 52, Q6_K 84 against 74).
+// Bound: the read of the weights (5.4-6.7 TB/s at 152064 x 3584).  Four tiles
+// in flight instead of two: 57 us against 52 (Q4_K).  Rows of more columns than the waves hold (MULTI) go in
+// chunks: a batch's tiles take one chunk after the other, the waves' sums
+// kept in LDS.
+constexpr int kVecs = 4, kBatch = 8, kMaxWaves = 16, kInFlight = 2;
+constexpr int kXRow = 264, kXWave = 9 * kXRow + 112;    // f16s: a row of 256, padded; a wave's rows, zeros and sums
+// floats of a tile's sums (16 more: the rows of four tiles in different banks)
+__host__ __device__ constexpr int lds_tile(int nw) { return nw * 64 + 16; }
+constexpr size_t gemv_lds(int nw)
+{
+    return sizeof(float) * 2 * kBatch * lds_tile(nw) + sizeof(_Float16) * kXWave * nw;
+}
+
+struct XOps {
+    h8_t f[8];
+    h8_t sx;
+    float inv;          // 1 / s of vector g
+};
+
+// The operands of a record's columns [c0, c0 + 256): a lane converts columns
+// 4 L .. + 3 of each vector, and the parts meet in LDS.
+template <class F>
+__device__ __forceinline__ void x_ops(XOps &o, const f4_t (&raw)[kVecs], _Float16 *lds, int nv, int cols, int c0)
+{
+    // row 2 v + part of the wave's LDS: the part's 256 f16s in operand order
+    // (step, g, 8); row 8: zeros, for the unused rows of A; then [v][part][8]
+    // of the sums
+    const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+    _Float16 *sxs = lds + 9 * kXRow;
+    const int k = lane >> 3, c = (lane & 7) * 4;        // the lane's step, columns c .. c + 3 of it
+    const int at = 32 * k + (F::kSplit ? (c & 15) * 2 + (c >> 4) * 4 : c);
+    *reinterpret_cast<h4_t *>(lds + 8 * kXRow + 4 * lane) = h4_t{0, 0, 0, 0};
+    o.inv = 1.0f;
+#pragma unroll
+    for (int v = 0; v < kVecs; v++)
+        if (v < nv) {
+            const f4_t a = c0 + 4 * lane < cols ? raw[v] : kZero;
+            float mx = fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3])));
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+            float s, inv;
+            x_scale(mx, s, inv);
+            o.inv = g == v ? inv : o.inv;
+            h4_t hi, lo;
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float t = a[i] * s;
+                _Float16 h, l;
+                x_split(t, h, l);
+                hi[x_pos<F>(i)] = h;
+                lo[x_pos<F>(i)] = l;
+                sum += t;
+            }
+            *reinterpret_cast<h4_t *>(lds + 2 * v * kXRow + at) = hi;
+            *reinterpret_cast<h4_t *>(lds + (2 * v + 1) * kXRow + at) = lo;
+            if constexpr (F::kMin) {
+                sum += __shfl_xor(sum, 1, 64);
+                sum += __shfl_xor(sum, 2, 64);
+                sum += __shfl_xor(sum, 4, 64);
+                _Float16 p0, p1, p2;
+                x_split3(sum * 0.015625f, p0, p1, p2);
+                if ((lane & 7) < 3) sxs[24 * v + 8 * (lane & 7) + k] = (lane & 7) == 0 ? p0 : (lane & 7) == 1 ? p1 : p2;
+            }
+        }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    constexpr int kC = 64 / kRB;           // lanes per row, 64 / kC partials each
-    const float4 *q = reinterpret_cast<const float4 *>(t + (lane % kRB) * 64 + (64 / kC) * (lane / kRB));
-    float s = 0.0f;
+    const bool on = (m >> 2) < nv && (F::kHalf || (m & 3) < 2);
+    const _Float16 *row = lds + (on ? 2 * (m >> 2) + (m & 1) : 8) * kXRow + 8 * g;
 #pragma unroll
-    for (int i = 0; i < 16 / kC; i++) {
-        const float4 v = q[i];
-        s += (v.x + v.y) + (v.z + v.w);
-    }
-#pragma unroll
-    for (int d = kRB; d < 64; d <<= 1) s += __shfl_xor(s, d, 64);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();       // the tile is free for the next batch
-    return s;
-}
-
-// Bytes 0..3 of a word as floats (v_cvt_f32_ubyte0..3).
-__device__ __forceinline__ float ub(uint32_t w, int t) { return (float)((w >> (8 * t)) & 0xffu); }
-
-// ---------------------------------------------------------------- Q6_K -----
-// Quarter qi of a row: block j = qi / 4, half h = (qi / 2) % 2, l0 = 16 (qi % 2).
-// Its 64 weights sit at 256 j + 128 h + 32 g + l, g = 0..3, l = l0 .. l0 + 15
-// (src/tensor/dequant.rs:203-214): group g takes the low nibble of
-// ql[64h + l] (g 0) / ql[64h + 32 + l] (g 1), the high nibbles (g 2, 3), and
-// bits 2g..2g+1 of qh[32h + l]; its scale is sc[8h + l0/16 + 2g].
-struct Q6Quarter {
-    uint4 a, b, c;      // ql[64h + l0 ..], ql[64h + 32 + l0 ..], qh[32h + l0 ..]
-    uint32_t s;         // byte g: sc[8h + l0/16 + 2g]
-    uint16_t d;
-};
-
-// Planes of a Q6_K matrix on the device (see the layout above); e indexes
-// quarters (row * 4nb + quarter), blocks are e / 4.
-struct Q6Planes {
-    const uint8_t *a, *b, *c;
-    const uint32_t *s;
-    const uint16_t *d;
-};
-
-// e < 2^28 (the upload limits a plane to 4 GB): 32-bit offsets from the
-// wave-uniform plane bases.
-__device__ __forceinline__ Q6Quarter q6_load(const Q6Planes &P, uint32_t e)
-{
-    Q6Quarter q;
-    q.a = ntl4(P.a + e * 16u);
-    q.b = ntl4(P.b + e * 16u);
-    q.c = ntl4(P.c + e * 16u);
-    q.s = __builtin_nontemporal_load(P.s + e);
-    q.d = __builtin_nontemporal_load(P.d + (e >> 2));
-    return q;
-}
-
-// sum over the quarter's four groups of scale_g * sum (u - 32) x.
-// xg[g][i] = x at the group's i-th weight, sx[g] = sum of xg[g].
-__device__ __forceinline__ float q6_dot(const Q6Quarter &q, const float (&xg)[4][16], const float (&sx)[4])
-{
-    float dot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t A[4] = {q.a.x, q.a.y, q.a.z, q.a.w};
-    const uint32_t B[4] = {q.b.x, q.b.y, q.b.z, q.b.w};
-    const uint32_t C[4] = {q.c.x, q.c.y, q.c.z, q.c.w};
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-        const uint32_t a = A[w], b = B[w], c = C[w];
-        const uint32_t u[4] = {(a & 0x0F0F0F0Fu) | ((c & 0x03030303u) << 4),
-                               (b & 0x0F0F0F0Fu) | ((c & 0x0C0C0C0Cu) << 2),
-                               ((a >> 4) & 0x0F0F0F0Fu) | (c & 0x30303030u),
-                               ((b >> 4) & 0x0F0F0F0Fu) | ((c >> 2) & 0x30303030u)};
-#pragma unroll
-        for (int g = 0; g < 4; g++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) dot[g] = fmaf(ub(u[g], t), xg[g][4 * w + t], dot[g]);
-    }
-    const float d = h2f(q.d);
-    float acc = 0.0f;
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const float scl = d * (float)(int8_t)(uint8_t)(q.s >> (8 * g));   // (d * scale), as the reference
-        acc = fmaf(scl, fmaf(-32.0f, sx[g], dot[g]), acc);
-    }
-    return acc;
-}
-
-__device__ __forceinline__ void q6_xslice(const float *x, int j, int h, int l0, float (&xg)[4][16], float (&sx)[4])
-{
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const float4 *p = reinterpret_cast<const float4 *>(x + 256 * j + 128 * h + 32 * g + l0);
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float4 v = p[i];
-            xg[g][4 * i] = v.x; xg[g][4 * i + 1] = v.y; xg[g][4 * i + 2] = v.z; xg[g][4 * i + 3] = v.w;
+    for (int ks = 0; ks < 8; ks++) {
+        h8_t h = *reinterpret_cast<const h8_t *>(row + 32 * ks);
+        if constexpr (F::kHalf) {
+            const h4_t z = {0, 0, 0, 0}, a = {h[0], h[1], h[2], h[3]}, b = {h[4], h[5], h[6], h[7]};
+            const h4_t c = m & 2 ? z : a, d = m & 2 ? b : z;
+            h = h8_t{c[0], c[1], c[2], c[3], d[0], d[1], d[2], d[3]};
         }
-#pragma unroll
-        for (int i = 0; i < 16; i++) s += xg[g][i];
-        sx[g] = s;
+        o.f[ks] = h;
     }
+    if constexpr (F::kMin)      // (g = 3, other rows: zeros)
+        o.sx = *reinterpret_cast<const h8_t *>((m & 3) == 0 && (m >> 2) < nv && g < 3 ? sxs + 24 * (m >> 2) + 8 * g
+                                                                                         : lds + 8 * kXRow);
 }
 
-// A block format whose lanes take quarters: 64 weights of block j at
-// 256 j + 128 h + 32 g + l0 + (0..15), g = 0..3 (Q6_K, Q3_K).
-struct Q6Fmt {
-    typedef Q6Planes Planes;
-    typedef Q6Quarter Unit;
-    static __device__ __forceinline__ Unit load(const Planes &P, uint32_t e) { return q6_load(P, e); }
-    static __device__ __forceinline__ float dot(const Unit &u, const float (&xg)[4][16], const float (&sx)[4])
-    {
-        return q6_dot(u, xg, sx);
-    }
-};
-
-// Rows of up to 16 blocks (cols <= 4096): one quarter per lane, x in
-// registers.  One NT-thread workgroup per CU stages x in LDS once; each wave
-// then takes a contiguous run of rows and keeps the loads of the next PF rows
-// in flight while it computes one (PF divides kRB, so the ring of row
-// buffers is indexed statically).
-template <class F, int kRB, int PF, int NT>
-__device__ __forceinline__ void quarter_rows_xreg(const typename F::Planes &P, const float *x, float *out, int rows,
-                                                  int nb, float *xs, float (*tiles)[kRB * 64])
+// A record's sum for the lane's row and vector, times s.
+template <class F> __device__ __forceinline__ float dot(const typename F::Item &it, const XOps &x)
 {
-    static_assert(kRB % PF == 0, "ring of PF row buffers, kRB rows per batch");
-    const int cols = 256 * nb;
-    for (int i = threadIdx.x; i < cols; i += NT) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (NT / 64);
-    const int gw = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    const int NQ = 4 * nb;
-    const bool act = lane < NQ;
-    const int qi = act ? lane : 0;
-    const int j = qi >> 2, h = (qi >> 1) & 1, l0 = (qi & 1) * 16;
-    float xg[4][16], sx[4];
-    q6_xslice(xs, j, h, l0, xg, sx);
-    const int rpw = (rows + nw - 1) / nw;
-    const int r0 = gw * rpw, r1 = min(rows, r0 + rpw);
-    if (r0 >= r1) return;
-    float *tile = tiles[threadIdx.x >> 6];
-    const uint32_t e1 = (uint32_t)(r1 - 1) * NQ + qi;
-    auto row_e = [&](int r) { return min((uint32_t)r * NQ + qi, e1); };   // past the run: its last row
-    typename F::Unit buf[PF];
+    float v = 0.0f;
+    f4_t D = kZero;
 #pragma unroll
-    for (int i = 0; i < PF; i++) buf[i] = F::load(P, row_e(r0 + i));
-    int rb = r0;
-    for (; rb + kRB <= r1; rb += kRB) {        // full batches
-        float part[kRB];
-#pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            const typename F::Unit nxt = F::load(P, row_e(rb + k + PF));
-            part[k] = act ? F::dot(buf[k % PF], xg, sx) : 0.0f;
-            buf[k % PF] = nxt;
+    for (int ks = 0; ks < 8; ks++) {
+        if constexpr (F::kHalf) {
+            const h4_t a = F::frag(it, ks, 0), b = F::frag(it, ks, 1);
+            D = mfma(x.f[ks], h8_t{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}, kZero);
+            v = fmaf(D[0] + D[1], F::sub(it, ks, 0), v);
+            v = fmaf(D[2] + D[3], F::sub(it, ks, 1), v);
+        } else {
+            D = mfma(x.f[ks], F::frag(it, ks), F::kChain ? D : kZero);
+            if constexpr (!F::kChain) v = fmaf(D[0] + D[1], F::sub(it, ks, 0), v);
         }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB) out[rb + lane] = v;
     }
-    if (rb < r1) {                             // the last, partial batch
-        float part[kRB];
+    if constexpr (F::kChain) v = D[0] + D[1];
+    if constexpr (F::kRecScale) v *= F::rec(it);
+    if constexpr (F::kMin) v = fmaf(mfma(x.sx, F::min_frag(it), kZero)[0], F::min_scale(it), v);
+    return v;
+}
+
+template <class F, bool MULTI>
+__global__ void __launch_bounds__(64 * kMaxWaves)
+qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, int np, int nv, int tiles, int tpb)
+{
+    extern __shared__ __align__(16) float red[];    // [2][batch] sums of a tile, then the waves' x
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6, ts = lds_tile(nw);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t0 = blockIdx.x * tpb, t1 = min(t0 + tpb, tiles);
+    if (t0 >= t1) return;
+    _Float16 *xl = reinterpret_cast<_Float16 *>(red + 2 * kBatch * ts) + kXWave * w;
+    XOps xo;
+    typename F::Item it[kInFlight];
+    // past the block's tiles or the row's records: the last one, not used
+    auto load = [&](int d, int t, int p) {
+        F::load(it[d], opaque(W + ((size_t)min(t, t1 - 1) * np + min(p, np - 1)) * F::kRec), lane);
+    };
+    auto start = [&](int t, int p) {        // (x first: loads return in order)
+        f4_t raw[kVecs];
 #pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            part[k] = 0.0f;
-            if (rb + k < r1 && act) part[k] = F::dot(buf[k % PF], xg, sx);   // rows rb .. r1-1 are in the ring
-            if (k + 1 < kRB && (k + 1) % PF == 0 && rb + k + 1 < r1) {
+        for (int v = 0; v < kVecs; v++)
+            raw[v] = *reinterpret_cast<const f4_t *>(x + (size_t)min(v, nv - 1) * cols + min(kPair * p + 4 * lane, cols - 4));
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i = 0; i < PF; i++) buf[i] = F::load(P, row_e(rb + k + 1 + i));
+        for (int d = 0; d < kInFlight; d++) load(d, t + d, p);
+        __builtin_amdgcn_sched_barrier(0);
+        x_ops<F>(xo, raw, xl, nv, cols, kPair * p);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (!MULTI) start(t0, w);
+    int buf = 0;
+    for (int tb = t0; tb < t1; tb += kBatch, buf ^= 1) {
+        const int nb = min(kBatch, t1 - tb);
+        float *rb = red + buf * kBatch * ts;
+        for (int c = 0; c < (MULTI ? np : 1); c += nw) {
+            const int p = c + w;
+            if (MULTI) start(tb, p);
+            for (int k0 = 0; k0 < nb; k0 += kInFlight) {
+                switch (k0 * 4 / kBatch) {
+                case 0: __builtin_amdgcn_s_setprio(3); break;
+                case 1: __builtin_amdgcn_s_setprio(2); break;
+                case 2: __builtin_amdgcn_s_setprio(1); break;
+                default: __builtin_amdgcn_s_setprio(0); break;
+                }
+#pragma unroll
+                for (int d = 0; d < kInFlight; d++) {       // (a tile past nb: not used)
+                    const int k = k0 + d;
+                    float v = dot<F>(it[d], xo) * xo.inv;
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(d, tb + k + kInFlight, p);
+                    float *q = rb + k * ts + w * 64 + lane;
+                    if (MULTI) {
+                        if (p >= np) v = 0.0f;
+                        if (c > 0) v += *q;
+                    }
+                    *q = v;
+                }
             }
         }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB && rb + lane < r1) out[rb + lane] = v;
-    }
-}
-template <int kRB, int PF, int NT>
-__global__ void __launch_bounds__(NT)
-q6k_gemv_xreg(Q6Planes P, const float *x, float *out, int rows, int nb)
-{
-    __shared__ float xs[4096];
-    __shared__ float tiles[NT / 64][kRB * 64];
-    quarter_rows_xreg<Q6Fmt, kRB, PF, NT>(P, x, out, rows, nb, xs, tiles);
-}
-
-// Any row length up to kMaxCols: x staged in LDS, lanes loop over quarters.
-template <class F>
-__device__ __forceinline__ void quarter_rows_lds(const typename F::Planes &P, const float *x, float *out, int rows,
-                                                 int nb, float *xs)
-{
-    const int cols = 256 * nb;
-    for (int i = threadIdx.x; i < cols; i += kGemvThreads) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (kGemvThreads / 64);
-    const int gw = blockIdx.x * (kGemvThreads / 64) + (threadIdx.x >> 6);
-    const int NQ = 4 * nb;
-    for (int r = gw; r < rows; r += nw) {
-        float v = 0.0f;
-        for (int qi = lane; qi < NQ; qi += 64) {
-            const int j = qi >> 2, h = (qi >> 1) & 1, l0 = (qi & 1) * 16;
-            float xg[4][16], sx[4];
-            q6_xslice(xs, j, h, l0, xg, sx);
-            v += F::dot(F::load(P, (uint32_t)r * NQ + qi), xg, sx);
-        }
-        v = wave_sum(v);
-        if (lane == 0) out[r] = v;
-    }
-}
-__global__ void __launch_bounds__(kGemvThreads)
-q6k_gemv_lds(Q6Planes P, const float *x, float *out, int rows, int nb)
-{
-    __shared__ float xs[kMaxCols];
-    quarter_rows_lds<Q6Fmt>(P, x, out, rows, nb, xs);
-}
-
-// ---------------------------------------------------------------- Q3_K -----
-// The GGUF layout (110 bytes: hmask[32], qs[64], scales[12], f16 d): weight
-// 128 n + 32 j + l has low bits (qs[32 n + l] >> 2 j) & 3, third bit
-// (hmask[l] >> (4 n + j)) & 1, value q = bits - 4, and scale (16 sub-blocks
-// of 16, 6 bits each, minus 32).  A quarter (n, l0) is the Q6_K quarter
-// (h = n, g = j).  The upload merges the three bits of a weight into a
-// nibble, u = q + 4 (the decode is then Q4_K's: 146 bytes per block on the
-// device for the file's 110, and about half the instructions per weight).
-// Planes, element e = 4 block + 2 n + l0 / 16:
-//   q: 32 bytes per quarter: byte k of the first 16 holds u of weight
-//   l0 + k of group 0 (low nibble) and group 1 (high), of the second 16
-//   groups 2 and 3; s: one word per quarter, byte j = the signed scale of
-//   group j; d: the f16 d per block.
-struct Q3Planes {
-    const uint8_t *q;
-    const uint32_t *s;
-    const uint16_t *d;
-};
-struct Q3Quarter {
-    uint4 a, b;
-    uint32_t s;
-    uint16_t d;
-};
-struct Q3Fmt {
-    typedef Q3Planes Planes;
-    typedef Q3Quarter Unit;
-    static __device__ __forceinline__ Unit load(const Planes &P, uint32_t e)
-    {
-        Unit u;
-        u.a = ntl4(P.q + e * 32u);
-        u.b = ntl4(P.q + e * 32u + 16u);
-        u.s = __builtin_nontemporal_load(P.s + e);
-        u.d = __builtin_nontemporal_load(P.d + (e >> 2));
-        return u;
-    }
-    // sum over the groups of (d * scale_j) * (sum u x - 4 sum x), u = q + 4
-    static __device__ __forceinline__ float dot(const Unit &u, const float (&xg)[4][16], const float (&sx)[4])
-    {
-        const uint32_t A[4] = {u.a.x, u.a.y, u.a.z, u.a.w}, B[4] = {u.b.x, u.b.y, u.b.z, u.b.w};
-        float dt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        __builtin_amdgcn_s_setprio(3);
+        // a wave adds four tiles of a vector at a time: vector v, row n is in
+        // lane 16 v + n
+        for (int u = w; u < nv * (kBatch / 4); u += nw) {
+            const int v = u / (kBatch / 4), rr = (u % (kBatch / 4)) * 64 + lane;
+            const uint32_t r = 16u * tb + rr;
+            const float *q = rb + (rr >> 4) * ts + v * 16 + (lane & 15);
+            float s = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const uint32_t v[4] = {A[w] & 0x0F0F0F0Fu, (A[w] >> 4) & 0x0F0F0F0Fu, B[w] & 0x0F0F0F0Fu,
-                                   (B[w] >> 4) & 0x0F0F0F0Fu};
+            for (int i = 0; i < kMaxWaves; i++)
+                if (i < nw) s += q[i * 64];
+            if (rr < 16 * nb && r < (uint32_t)rows) out[(size_t)v * rows + r] = s;
+        }
+    }
+}
+
+// ------------------------------------------- more vectors, up to 32 (GEMM) ---
+// VT tiles of 16 vectors: row m of A's tile vt is vector 16 vt + m, hi and lo
+// two MFMAs into one D, whose rows are the vectors.
+//
+// A block of 8 waves (one per CU, 2 waves per SIMD: 256 registers each) takes
+// up to 8 RT tiles of 16 rows at a time, RT to a wave, through all columns.
+// The x of a record is converted once per block into LDS (each wave a step of
+// all vectors; two buffers, one barrier per record) and read from there for
+// two or three groups of the wave's tiles; a group's registers are loaded
+// again, for the next record, as soon as it has been used.  (x of 32 vectors
+// in registers for all columns would fill the CU's register file.)
+// Bound: the chain of a step in each wave (unpack, two MFMAs, additions) at
+// two waves per SIMD; VALU issue is 48% at 16 vectors.  Holding x in
+// registers as the kernel above does (up to 8 vectors in 128 registers, 16
+// with spills) took 74 us at 8 and 87 at 16 (Q4_K 152064 x 3584) where this
+// takes 74 and 77, and 158 for 32 in two passes where this takes 115.
+constexpr int kGemmWaves = 8;
+template <class F, int VT> constexpr int kXBuf = VT * (2 * 8 * 512 + (F::kMin ? 512 : 0));     // f16s of a record's x
+
+template <class F, int VT, int N>
+__device__ __forceinline__ void group(const typename F::Item *it, const _Float16 *xb, float (*acc)[VT][4])
+{
+    const int lane = threadIdx.x & 63;
+    xb += 8 * lane;
+    float sum[N][VT][4] = {};   // of the record: shorter chains of additions
+    h8_t nh[VT], no[VT];        // the next step's x, read a step ahead
+    auto read = [&](int ks) {
+#pragma unroll
+        for (int v = 0; v < VT; v++) {
+            nh[v] = *reinterpret_cast<const h8_t *>(xb + (16 * v + ks) * 512);
+            no[v] = *reinterpret_cast<const h8_t *>(xb + (16 * v + 8 + ks) * 512);
+        }
+    };
+    read(0);
+#pragma unroll
+    for (int ks = 0; ks < 8; ks++) {
+        h8_t xh[VT], xo[VT];
+#pragma unroll
+        for (int v = 0; v < VT; v++) { xh[v] = nh[v]; xo[v] = no[v]; }
+        if (ks < 7) read(ks + 1);
+#pragma unroll
+        for (int r = 0; r < N; r++)
+#pragma unroll
+            for (int i = 0; i < (F::kHalf ? 2 : 1); i++) {
+                const float s = F::sub(it[r], ks, i);
+#pragma unroll
+                for (int v = 0; v < VT; v++) {
+                    f4_t D;
+                    if constexpr (F::kHalf) {
+                        const h4_t b = F::frag(it[r], ks, i);
+                        D = mfma(h4_t{xh[v][4 * i], xh[v][4 * i + 1], xh[v][4 * i + 2], xh[v][4 * i + 3]}, b, kZero);
+                        D = mfma(h4_t{xo[v][4 * i], xo[v][4 * i + 1], xo[v][4 * i + 2], xo[v][4 * i + 3]}, b, D);
+                    } else {
+                        const h8_t b = F::frag(it[r], ks);
+                        D = mfma(xh[v], b, kZero);
+                        D = mfma(xo[v], b, D);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; j++) sum[r][v][j] = fmaf(D[j], s, sum[r][v][j]);
+                }
+            }
+        // a step's sums are done here (else the steps of a record are mixed
+        // until the registers spill)
+        if (VT == 2 || F::kHalf) {
+#pragma unroll
+            for (int r = 0; r < N; r++)
+#pragma unroll
+                for (int v = 0; v < VT; v++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) asm volatile("" : "+v"(sum[r][v][j]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+        const float s = F::rec(it[r]);
+#pragma unroll
+        for (int v = 0; v < VT; v++)
 #pragma unroll
             for (int j = 0; j < 4; j++)
-#pragma unroll
-                for (int t = 0; t < 4; t++) dt[j] = fmaf(ub(v[j], t), xg[j][4 * w + t], dt[j]);
-        }
-        const float d = h2f(u.d);
-        float acc = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float scl = d * (float)(int8_t)(uint8_t)(u.s >> (8 * j));   // (d * sc), as the reference
-            acc = fmaf(scl, fmaf(-4.0f, sx[j], dt[j]), acc);
-        }
-        return acc;
+                acc[r][v][j] = F::kRecScale ? fmaf(sum[r][v][j], s, acc[r][v][j]) : acc[r][v][j] + sum[r][v][j];
     }
-};
-constexpr int kRB3 = 8, kPF3 = 2, kNT3 = 768;   // Q3_K: the Q6_K structure
-template <int kRB, int PF, int NT>
-__global__ void __launch_bounds__(NT)
-q3k_gemv_xreg(Q3Planes P, const float *x, float *out, int rows, int nb)
-{
-    __shared__ float xs[4096];
-    __shared__ float tiles[NT / 64][kRB * 64];
-    quarter_rows_xreg<Q3Fmt, kRB, PF, NT>(P, x, out, rows, nb, xs, tiles);
-}
-__global__ void __launch_bounds__(kGemvThreads)
-q3k_gemv_lds(Q3Planes P, const float *x, float *out, int rows, int nb)
-{
-    __shared__ float xs[kMaxCols];
-    quarter_rows_lds<Q3Fmt>(P, x, out, rows, nb, xs);
-}
-
-// ---------------------------------------------------------------- Q8_0 -----
-// Half block hb of a row: block hb / 2, weights 32 (hb / 2) + 16 (hb % 2) .. + 15.
-__device__ __forceinline__ float q8_dot(uint4 q, uint16_t d16, const float *xs16, float sx)
-{
-    const uint32_t W[4] = {q.x ^ 0x80808080u, q.y ^ 0x80808080u, q.z ^ 0x80808080u, q.w ^ 0x80808080u};
-    float dot = 0.0f;
+    if constexpr (F::kMin) {
 #pragma unroll
-    for (int w = 0; w < 4; w++)
+        for (int v = 0; v < VT; v++) {
+            const h8_t sx = *reinterpret_cast<const h8_t *>(xb + (16 * VT + v) * 512);
 #pragma unroll
-        for (int t = 0; t < 4; t++) dot = fmaf(ub(W[w], t), xs16[4 * w + t], dot);
-    return h2f(d16) * fmaf(-128.0f, sx, dot);
-}
-
-// Measured on MI355X at the Qwen2.5-7B shape (same box, interleaved runs):
-// Q6_K 768 threads (12 waves per CU, 157 VGPRs), 2 rows in flight, 8 rows
-// per reduction batch: 77-78 us; one row in flight at 1024 threads: 88-89 us;
-// 4 rows in flight (211 VGPRs, 8 waves): 84 us.  Q8_0: 4 rows per batch
-// (8 spill at 1024 threads with one row in flight).
-constexpr int kRB6 = 8, kPF6 = 2, kNT6 = 768;   // Q6_K: rows per batch, rows in flight, threads
-constexpr int kRB8 = 8, kPF8 = 2, kNT8 = 768;   // Q8_0: the same structure
-constexpr int kQ8Halves = 4;            // half blocks per lane on the register path (cols <= 4096)
-
-// One row's quants and scales for a lane (kQ8Halves half blocks).
-struct Q8Row {
-    uint4 q[kQ8Halves];
-    uint16_t d[kQ8Halves];
-};
-
-// As q6k_gemv_xreg: x (64 values per lane) in registers, PF rows in flight.
-template <int kRB, int PF, int NT>
-__global__ void __launch_bounds__(NT)
-q80_gemv_xreg(const uint8_t *bits, const uint16_t *dq, const float *x, float *out, int rows, int nb)
-{
-    static_assert(kRB % PF == 0, "ring of PF row buffers, kRB rows per batch");
-    __shared__ float xs[4096];
-    __shared__ float tiles[NT / 64][kRB * 64];
-    const int cols = 32 * nb;
-    for (int i = threadIdx.x; i < cols; i += NT) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (NT / 64);
-    const int gw = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    const int nh = 2 * nb;
-    float xv[kQ8Halves][16], sx[kQ8Halves];
-    bool act[kQ8Halves];
-    int hb[kQ8Halves];
+            for (int r = 0; r < N; r++) {
+                const f4_t D = mfma(sx, F::min_frag(it[r]), kZero);
+                const float s = F::min_scale(it[r]);
 #pragma unroll
-    for (int k = 0; k < kQ8Halves; k++) {
-        act[k] = lane + 64 * k < nh;
-        hb[k] = act[k] ? lane + 64 * k : 0;
-        const float4 *p = reinterpret_cast<const float4 *>(xs + 16 * hb[k]);
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float4 v = p[i];
-            xv[k][4 * i] = v.x; xv[k][4 * i + 1] = v.y; xv[k][4 * i + 2] = v.z; xv[k][4 * i + 3] = v.w;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; i++) s += xv[k][i];
-        sx[k] = s;
-    }
-    const int rpw = (rows + nw - 1) / nw;
-    const int r0 = gw * rpw, r1 = min(rows, r0 + rpw);
-    if (r0 >= r1) return;
-    float *tile = tiles[threadIdx.x >> 6];
-    auto load = [&](int r) {                   // rows past the run read its last row
-        const uint32_t rr = (uint32_t)min(r, r1 - 1);
-        Q8Row w;
-#pragma unroll
-        for (int k = 0; k < kQ8Halves; k++) {
-            const uint32_t e = rr * (uint32_t)nh + (uint32_t)hb[k];
-            w.q[k] = ntl4(bits + e * 16u);
-            w.d[k] = __builtin_nontemporal_load(dq + (e >> 1));
-        }
-        return w;
-    };
-    auto dot = [&](const Q8Row &w) {
-        float v = 0.0f;
-#pragma unroll
-        for (int k = 0; k < kQ8Halves; k++)
-            if (act[k]) v += q8_dot(w.q[k], w.d[k], xv[k], sx[k]);
-        return v;
-    };
-    Q8Row buf[PF];
-#pragma unroll
-    for (int i = 0; i < PF; i++) buf[i] = load(r0 + i);
-    int rb = r0;
-    for (; rb + kRB <= r1; rb += kRB) {        // full batches
-        float part[kRB];
-#pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            const Q8Row nxt = load(rb + k + PF);
-            part[k] = dot(buf[k % PF]);
-            buf[k % PF] = nxt;
-        }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB) out[rb + lane] = v;
-    }
-    if (rb < r1) {                             // the last, partial batch
-        float part[kRB];
-#pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            part[k] = rb + k < r1 ? dot(buf[k % PF]) : 0.0f;
-            if (k + 1 < kRB && (k + 1) % PF == 0 && rb + k + 1 < r1) {
-#pragma unroll
-                for (int i = 0; i < PF; i++) buf[i] = load(rb + k + 1 + i);
+                for (int j = 0; j < 4; j++) acc[r][v][j] = fmaf(D[j], s, acc[r][v][j]);
             }
         }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB && rb + lane < r1) out[rb + lane] = v;
     }
+    // The additions are done here: put off past the branches that follow they
+    // keep the products of all steps in registers.
+#pragma unroll
+    for (int r = 0; r < N; r++)
+#pragma unroll
+        for (int v = 0; v < VT; v++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[r][v][j]));
 }
 
-__global__ void __launch_bounds__(kGemvThreads)
-q80_gemv_lds(const uint8_t *bits, const uint16_t *dq, const float *x, float *out, int rows, int nb)
+template <class F, int VT, int RT>
+__global__ void __launch_bounds__(64 * kGemmWaves)
+qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, int np, int B, int per, int tiles, int tpb)
 {
-    __shared__ float xs[kMaxCols];
-    const int cols = 32 * nb;
-    for (int i = threadIdx.x; i < cols; i += kGemvThreads) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (kGemvThreads / 64);
-    const int gw = blockIdx.x * (kGemvThreads / 64) + (threadIdx.x >> 6);
-    for (int r = gw; r < rows; r += nw) {
-        float v = 0.0f;
-        for (int hbk = lane; hbk < 2 * nb; hbk += 64) {
-            const size_t blk = (size_t)r * nb + (hbk >> 1);
-            const uint4 q = ntl4(bits + blk * 32 + 16 * (hbk & 1));
-            const float *xp = xs + 16 * hbk;
-            float s = 0.0f;
-            for (int i = 0; i < 16; i++) s += xp[i];
-            v += q8_dot(q, __builtin_nontemporal_load(dq + blk), xp, s);
-        }
-        v = wave_sum(v);
-        if (lane == 0) out[r] = v;
-    }
-}
+    // RT > 1: the wave's tiles in groups of N; RT = 1: two records of its tile
+    constexpr int N = RT <= 3 ? (RT + 1) / 2 : VT == 2 ? 2 : (RT + 1) / 2, NI = RT > 1 ? RT : 2;
+    __shared__ __align__(16) _Float16 xs[2][kXBuf<F, VT>];
+    __shared__ float sc[VT * 16], si[VT * 16];
+    const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int v0 = blockIdx.y * per, nv = min(per, B - v0);
+    const int t0 = blockIdx.x * tpb, t1 = min(t0 + tpb, tiles);
+    if (t0 >= t1) return;
+    x += (size_t)v0 * cols;
+    out += (size_t)v0 * rows;
 
-// ---------------------------------------------------------- Q4_0 / Q4_1 -----
-// Block j of a row (src/tensor/dequant.rs:26-54): byte l of its 16 bytes of
-// nibbles holds weight 32 j + l (low nibble) and 32 j + 16 + l (high).
-// Q4_0: w = (q - 8) d; Q4_1: w = q d + m.  Planes: qs, 16 bytes per block;
-// Q4_0 the f16 d per block, Q4_1 one word per block, d | m << 16.
-struct Q4Planes {
-    const uint8_t *qs;
-    const uint16_t *d;      // Q4_0
-    const uint32_t *dm;     // Q4_1
-};
-constexpr int kQ4Blocks = 2;            // blocks per lane on the register path (cols <= 4096)
-constexpr int kRB4 = 8, kPF4 = 4, kNT4 = 768;   // rows per batch, rows in flight, threads
-
-template <bool Q41>
-__device__ __forceinline__ uint32_t q4_dm(const Q4Planes &P, uint32_t blk)
-{
-    return Q41 ? __builtin_nontemporal_load(P.dm + blk) : (uint32_t)__builtin_nontemporal_load(P.d + blk);
-}
-// Q4_0: d (sum q x - 8 sum x); Q4_1: d sum q x + m sum x.  xv: the block's
-// 32 values of x, sx their sum.
-template <bool Q41>
-__device__ __forceinline__ float q4_dot(uint4 q, uint32_t dm, const float *xv, float sx)
-{
-    const uint32_t W[4] = {q.x, q.y, q.z, q.w};
-    float lo = 0.0f, hi = 0.0f;
+    typename F::Item it[NI];
+    f4_t raw[2 * VT];
+    const float *xv[VT];
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
-        const uint32_t a = W[w] & 0x0F0F0F0Fu, b = (W[w] >> 4) & 0x0F0F0F0Fu;
+    for (int v = 0; v < VT; v++) xv[v] = x + (size_t)min(16 * v + m, nv - 1) * cols + (F::kSplit ? 4 * g : 8 * g);
+    auto xload = [&](int p) {       // step w of record p
+        const int c = min(kPair * p + 32 * w, cols - 32);
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            lo = fmaf(ub(a, t), xv[4 * w + t], lo);
-            hi = fmaf(ub(b, t), xv[16 + 4 * w + t], hi);
+        for (int v = 0; v < VT; v++) {
+            raw[2 * v] = *reinterpret_cast<const f4_t *>(xv[v] + c);
+            raw[2 * v + 1] = *reinterpret_cast<const f4_t *>(xv[v] + c + (F::kSplit ? 16 : 4));
         }
-    }
-    const float d = h2f((uint16_t)(dm & 0xffffu));
-    if (Q41) return fmaf(d, lo + hi, h2f((uint16_t)(dm >> 16)) * sx);
-    return d * fmaf(-8.0f, sx, lo + hi);
-}
-
-// As q80_gemv_xreg: kQ4Blocks blocks per lane, x (64 values) in registers,
-// PF rows in flight.
-template <bool Q41, int kRB, int PF, int NT>
-__global__ void __launch_bounds__(NT)
-q4_gemv_xreg(Q4Planes P, const float *x, float *out, int rows, int nb)
-{
-    static_assert(kRB % PF == 0, "ring of PF row buffers, kRB rows per batch");
-    __shared__ float xs[4096];
-    __shared__ float tiles[NT / 64][kRB * 64];
-    const int cols = 32 * nb;
-    for (int i = threadIdx.x; i < cols; i += NT) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (NT / 64);
-    const int gw = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    float xv[kQ4Blocks][32], sx[kQ4Blocks];
-    bool act[kQ4Blocks];
-    int bk[kQ4Blocks];
-#pragma unroll
-    for (int k = 0; k < kQ4Blocks; k++) {
-        act[k] = lane + 64 * k < nb;
-        bk[k] = act[k] ? lane + 64 * k : 0;
-        const float4 *p = reinterpret_cast<const float4 *>(xs + 32 * bk[k]);
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float4 v = p[i];
-            xv[k][4 * i] = v.x; xv[k][4 * i + 1] = v.y; xv[k][4 * i + 2] = v.z; xv[k][4 * i + 3] = v.w;
-        }
-#pragma unroll
-        for (int i = 0; i < 32; i++) s += xv[k][i];
-        sx[k] = s;
-    }
-    const int rpw = (rows + nw - 1) / nw;
-    const int r0 = gw * rpw, r1 = min(rows, r0 + rpw);
-    if (r0 >= r1) return;
-    float *tile = tiles[threadIdx.x >> 6];
-    struct Row { uint4 q[kQ4Blocks]; uint32_t dm[kQ4Blocks]; };
-    auto load = [&](int r) {                   // rows past the run read its last row
-        const uint32_t rr = (uint32_t)min(r, r1 - 1);
-        Row w;
-#pragma unroll
-        for (int k = 0; k < kQ4Blocks; k++) {
-            const uint32_t e = rr * (uint32_t)nb + (uint32_t)bk[k];
-            w.q[k] = ntl4(P.qs + e * 16u);
-            w.dm[k] = q4_dm<Q41>(P, e);
-        }
-        return w;
     };
-    auto dot = [&](const Row &w) {
-        float v = 0.0f;
+    float s[VT];
+    auto xput = [&](int p) {
+        _Float16 *b = xs[p & 1] + 8 * lane;
 #pragma unroll
-        for (int k = 0; k < kQ4Blocks; k++)
-            if (act[k]) v += q4_dot<Q41>(w.q[k], w.dm[k], xv[k], sx[k]);
-        return v;
-    };
-    Row buf[PF];
+        for (int v = 0; v < VT; v++) {
+            const bool in = 16 * v + m < nv && kPair * p + 32 * w < cols;
+            h8_t hi, lo;
+            float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < PF; i++) buf[i] = load(r0 + i);
-    int rb = r0;
-    for (; rb + kRB <= r1; rb += kRB) {        // full batches
-        float part[kRB];
+            for (int h = 0; h < 2; h++)
 #pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            const Row nxt = load(rb + k + PF);
-            part[k] = dot(buf[k % PF]);
-            buf[k % PF] = nxt;
-        }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB) out[rb + lane] = v;
-    }
-    if (rb < r1) {                             // the last, partial batch
-        float part[kRB];
-#pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            part[k] = rb + k < r1 ? dot(buf[k % PF]) : 0.0f;
-            if (k + 1 < kRB && (k + 1) % PF == 0 && rb + k + 1 < r1) {
-#pragma unroll
-                for (int i = 0; i < PF; i++) buf[i] = load(rb + k + 1 + i);
+                for (int i = 0; i < 4; i++) {
+                    const float t = in ? raw[2 * v + h][i] * s[v] : 0.0f;
+                    _Float16 a, c;
+                    x_split(t, a, c);
+                    hi[4 * h + x_pos<F>(i)] = a;
+                    lo[4 * h + x_pos<F>(i)] = c;
+                    sum += t;
+                }
+            *reinterpret_cast<h8_t *>(b + (16 * v + w) * 512) = hi;
+            *reinterpret_cast<h8_t *>(b + (16 * v + 8 + w) * 512) = lo;
+            if constexpr (F::kMin) {        // lanes 16 g + m hold part g of the sum over the step
+                sum += __shfl_xor(sum, 16, 64);
+                sum += __shfl_xor(sum, 32, 64);
+                _Float16 a0, a1, a2;
+                x_split3(sum * 0.015625f, a0, a1, a2);
+                b[(16 * VT + v) * 512 + w] = g == 0 ? a0 : g == 1 ? a1 : g == 2 ? a2 : (_Float16)0.0f;
             }
         }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB && rb + lane < r1) out[rb + lane] = v;
-    }
-}
+    };
+    auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
 
-template <bool Q41>
-__global__ void __launch_bounds__(kGemvThreads)
-q4_gemv_lds(Q4Planes P, const float *x, float *out, int rows, int nb)
-{
-    __shared__ float xs[kMaxCols];
-    const int cols = 32 * nb;
-    for (int i = threadIdx.x; i < cols; i += kGemvThreads) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (kGemvThreads / 64);
-    const int gw = blockIdx.x * (kGemvThreads / 64) + (threadIdx.x >> 6);
-    for (int r = gw; r < rows; r += nw) {
-        float v = 0.0f;
-        for (int b = lane; b < nb; b += 64) {
-            const uint32_t e = (uint32_t)r * (uint32_t)nb + (uint32_t)b;
-            const float *xp = xs + 32 * b;
-            float s = 0.0f;
-            for (int i = 0; i < 32; i++) s += xp[i];
-            v += q4_dot<Q41>(ntl4(P.qs + e * 16u), q4_dm<Q41>(P, e), xp, s);
-        }
-        v = wave_sum(v);
-        if (lane == 0) out[r] = v;
-    }
-}
-
-// ------------------------------------------------------- Q4_K / Q5_K -----
-// Step s of block j (src/tensor/dequant.rs:149-196, a "pair" here) holds the
-// 64 weights 256 j + 64 s + l (sub-block 2s: low nibbles of qs[32 s + l])
-// and 256 j + 64 s + 32 + l (sub-block 2s + 1: high nibbles), l = 0..31;
-// Q5_K adds bit 2s / 2s + 1 of qh[l] as 16.  w = (d * sc) * q - dmin * m.
-// Planes (element e = 4 j + s of a row; rows of 4 nb pairs):
-//   qs: 32 bytes per pair; h (Q5_K): two words per pair, bit l = the fifth
-//   bit of weight l of sub-block 2s / 2s + 1; sm: one word per pair, bytes
-//   sc(2s), m(2s), sc(2s + 1), m(2s + 1); dd: one word per block, d | dmin << 16.
-struct KPlanes {
-    const uint8_t *qs;
-    const uint2 *h;
-    const uint32_t *sm;
-    const uint32_t *dd;
-};
-struct KPair {
-    uint4 a, b;         // qs[32 s .. 32 s + 15], qs[32 s + 16 .. 32 s + 31]
-    uint2 h;
-    uint32_t sm, dd;
-};
-template <bool Q5>
-__device__ __forceinline__ KPair kq_load(const KPlanes &P, uint32_t e)
-{
-    KPair q;
-    q.a = ntl4(P.qs + e * 32u);
-    q.b = ntl4(P.qs + e * 32u + 16u);
-    q.h = Q5 ? ntl2(P.h + e) : make_uint2(0u, 0u);
-    q.sm = __builtin_nontemporal_load(P.sm + e);
-    q.dd = __builtin_nontemporal_load(P.dd + (e >> 2));
-    return q;
-}
-// Bits 0..3 of n to bit 4 of bytes 0..3.
-__device__ __forceinline__ uint32_t kq_hi4(uint32_t n) { return ((n * 0x00204081u) & 0x01010101u) << 4; }
-
-// (d sc_A) sum qA x - (dmin m_A) sum x + the same for sub-block B; xa / xb
-// the pair's x, sa / sb their sums.
-template <bool Q5>
-__device__ __forceinline__ float kq_dot(const KPair &q, const float (&xa)[32], const float (&xb)[32], float sa, float sb)
-{
-    const uint32_t W[8] = {q.a.x, q.a.y, q.a.z, q.a.w, q.b.x, q.b.y, q.b.z, q.b.w};
-    float da = 0.0f, db = 0.0f;
+    bool first = true;
+    const int rounds = (t1 - t0 + kGemmWaves * RT - 1) / (kGemmWaves * RT);
+    for (int rd = 0; rd < rounds; rd++) {
+        // the round's tiles, spread evenly over the waves
+        const int ra = t0 + (int)((long)(t1 - t0) * rd / rounds), nt = t0 + (int)((long)(t1 - t0) * (rd + 1) / rounds) - ra;
+        const int q = nt / kGemmWaves, rem = nt - q * kGemmWaves;
+        const int cnt = q + (w < rem), tw = ra + w * q + min(w, rem);
+        auto load = [&](int i, int r, int p) {      // past the wave's tiles or the records: the last, not used
+            F::load(it[i], opaque(W + ((size_t)min(tw + r, t1 - 1) * np + min(p, np - 1)) * F::kRec), lane);
+        };
+        xload(0);
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        uint32_t lo = W[k] & 0x0F0F0F0Fu, hi = (W[k] >> 4) & 0x0F0F0F0Fu;
-        if (Q5) {
-            lo |= kq_hi4((q.h.x >> (4 * k)) & 0xFu);
-            hi |= kq_hi4((q.h.y >> (4 * k)) & 0xFu);
-        }
+        for (int i = 0; i < NI; i++) load(i, RT > 1 ? i : 0, RT > 1 ? 0 : i);
+        if (first) {        // the scale of each vector, from all its columns
+            for (int v = w; v < 16 * VT; v += kGemmWaves) {
+                float mx = 0.0f;
+                if (v < nv) {
+                    const float *p = x + (size_t)v * cols;
+                    for (int c = 4 * lane; c < cols; c += 256) {
+                        const f4_t a = *reinterpret_cast<const f4_t *>(p + c);
+                        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))));
+                    }
+                }
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            da = fmaf(ub(lo, t), xa[4 * k + t], da);
-            db = fmaf(ub(hi, t), xb[4 * k + t], db);
-        }
-    }
-    const float d = h2f((uint16_t)(q.dd & 0xffffu)), dmin = h2f((uint16_t)(q.dd >> 16));
-    const float d1 = d * (float)(q.sm & 0xffu), mb1 = dmin * (float)((q.sm >> 8) & 0xffu);     // as the reference
-    const float d2 = d * (float)((q.sm >> 16) & 0xffu), mb2 = dmin * (float)(q.sm >> 24);
-    return fmaf(d1, da, fmaf(-mb1, sa, fmaf(d2, db, -mb2 * sb)));
-}
-__device__ __forceinline__ void kq_xslice(const float *x, int j, int st, float (&xa)[32], float (&xb)[32],
-                                          float *sa, float *sb)
-{
-    const float4 *pa = reinterpret_cast<const float4 *>(x + 256 * j + 64 * st);
-    const float4 *pb = reinterpret_cast<const float4 *>(x + 256 * j + 64 * st + 32);
-    float s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float4 u = pa[i], v = pb[i];
-        xa[4 * i] = u.x; xa[4 * i + 1] = u.y; xa[4 * i + 2] = u.z; xa[4 * i + 3] = u.w;
-        xb[4 * i] = v.x; xb[4 * i + 1] = v.y; xb[4 * i + 2] = v.z; xb[4 * i + 3] = v.w;
-    }
-#pragma unroll
-    for (int i = 0; i < 32; i++) { s1 += xa[i]; s2 += xb[i]; }
-    *sa = s1;
-    *sb = s2;
-}
-
-// As q6k_gemv_xreg, a pair per lane (rows of up to 16 blocks).
-template <bool Q5, int kRB, int PF, int NT>
-__global__ void __launch_bounds__(NT)
-kq_gemv_xreg(KPlanes P, const float *x, float *out, int rows, int nb)
-{
-    static_assert(kRB % PF == 0, "ring of PF row buffers, kRB rows per batch");
-    __shared__ float xs[4096];
-    __shared__ float tiles[NT / 64][kRB * 64];
-    const int cols = 256 * nb;
-    for (int i = threadIdx.x; i < cols; i += NT) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (NT / 64);
-    const int gw = blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    const int NQ = 4 * nb;
-    const bool act = lane < NQ;
-    const int qi = act ? lane : 0;
-    float xa[32], xb[32], sa, sb;
-    kq_xslice(xs, qi >> 2, qi & 3, xa, xb, &sa, &sb);
-    const int rpw = (rows + nw - 1) / nw;
-    const int r0 = gw * rpw, r1 = min(rows, r0 + rpw);
-    if (r0 >= r1) return;
-    float *tile = tiles[threadIdx.x >> 6];
-    const uint32_t e1 = (uint32_t)(r1 - 1) * NQ + qi;
-    auto row_e = [&](int r) { return min((uint32_t)r * NQ + qi, e1); };   // past the run: its last row
-    KPair buf[PF];
-#pragma unroll
-    for (int i = 0; i < PF; i++) buf[i] = kq_load<Q5>(P, row_e(r0 + i));
-    int rb = r0;
-    for (; rb + kRB <= r1; rb += kRB) {
-        float part[kRB];
-#pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            const KPair nxt = kq_load<Q5>(P, row_e(rb + k + PF));
-            part[k] = act ? kq_dot<Q5>(buf[k % PF], xa, xb, sa, sb) : 0.0f;
-            buf[k % PF] = nxt;
-        }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB) out[rb + lane] = v;
-    }
-    if (rb < r1) {
-        float part[kRB];
-#pragma unroll
-        for (int k = 0; k < kRB; k++) {
-            part[k] = 0.0f;
-            if (rb + k < r1 && act) part[k] = kq_dot<Q5>(buf[k % PF], xa, xb, sa, sb);
-            if (k + 1 < kRB && (k + 1) % PF == 0 && rb + k + 1 < r1) {
-#pragma unroll
-                for (int i = 0; i < PF; i++) buf[i] = kq_load<Q5>(P, row_e(rb + k + 1 + i));
+                for (int d = 1; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+                float a, b;
+                x_scale(mx, a, b);
+                if (lane == 0) { sc[v] = a; si[v] = b; }
             }
+            sync();
+            first = false;
+#pragma unroll
+            for (int v = 0; v < VT; v++) s[v] = sc[16 * v + m];
         }
-        const float v = rows_sum<kRB>(part, tile);
-        if (lane < kRB && rb + lane < r1) out[rb + lane] = v;
+        float acc[RT][VT][4] = {};
+        xput(0);
+        xload(1);
+        sync();
+        for (int p = 0; p < np; p += RT > 1 ? 1 : 2) {
+            const _Float16 *xb = xs[p & 1];
+            __builtin_amdgcn_s_setprio(3);
+            __builtin_amdgcn_sched_barrier(0);
+            group<F, VT, N>(it, xb, acc);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < N; i++) load(i, i, p + (RT > 1 ? 1 : 2));
+            xput(p + 1);
+            xload(p + 2);
+            if constexpr (RT > 1) {
+#pragma unroll
+                for (int r = N; r < RT; r += N) {
+                    constexpr int M = RT % N;       // the last group's, if it is smaller
+                    if (r == N) __builtin_amdgcn_s_setprio(1);
+                    else __builtin_amdgcn_s_setprio(0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (M == 0 || r + N <= RT) group<F, VT, N>(it + r, xb, acc + r);
+                    else group<F, VT, M ? M : 1>(it + r, xb, acc + r);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = r; i < r + N; i++)
+                        if (i < RT) load(i, i, p + 1);
+                }
+            } else {
+                sync();
+                float t[1][VT][4] = {};         // (past the last record: not used)
+                __builtin_amdgcn_sched_barrier(0);
+                group<F, VT, 1>(it + 1, xs[1], t);
+                __builtin_amdgcn_sched_barrier(0);
+                load(1, 0, p + 3);
+#pragma unroll
+                for (int v = 0; v < VT; v++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[0][v][j] += p + 1 < np ? t[0][v][j] : 0.0f;
+                xput(p + 2);
+                xload(p + 3);
+            }
+            sync();
+        }
+#pragma unroll
+        for (int v = 0; v < VT; v++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int vec = 16 * v + 4 * g + j;
+                const float inv = si[vec];
+#pragma unroll
+                for (int r = 0; r < RT; r++) {
+                    const uint32_t row = 16u * (tw + r) + m;
+                    if (r < cnt && vec < nv && row < (uint32_t)rows)
+                        __builtin_nontemporal_store(acc[r][v][j] * inv, out + (size_t)vec * rows + row);
+                }
+            }
     }
 }
 
-template <bool Q5>
-__global__ void __launch_bounds__(kGemvThreads)
-kq_gemv_lds(KPlanes P, const float *x, float *out, int rows, int nb)
+// GGUF blocks of rows [16 t0, 16 (t0 + tiles)) of the matrix (raw, nb blocks
+// of F::kBlock bytes per row, rows_here of them given) to records; one lane
+// of a record per thread.
+template <class F>
+__global__ void __launch_bounds__(256) repack_kernel(const uint8_t *raw, uint8_t *W, int rows_here, int nb, int np, int tiles)
 {
-    __shared__ float xs[kMaxCols];
-    const int cols = 256 * nb;
-    for (int i = threadIdx.x; i < cols; i += kGemvThreads) xs[i] = x[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const int nw = gridDim.x * (kGemvThreads / 64);
-    const int gw = blockIdx.x * (kGemvThreads / 64) + (threadIdx.x >> 6);
-    const int NQ = 4 * nb;
-    for (int r = gw; r < rows; r += nw) {
-        float v = 0.0f;
-        for (int qi = lane; qi < NQ; qi += 64) {
-            float xa[32], xb[32], sa, sb;
-            kq_xslice(xs, qi >> 2, qi & 3, xa, xb, &sa, &sb);
-            v += kq_dot<Q5>(kq_load<Q5>(P, (uint32_t)r * NQ + qi), xa, xb, sa, sb);
-        }
-        v = wave_sum(v);
-        if (lane == 0) out[r] = v;
-    }
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const int lane = (int)(i & 63);
+    const size_t rec = i >> 6;
+    if (rec >= (size_t)tiles * np) return;
+    const int t = (int)(rec / np), p = (int)(rec - (size_t)t * np);
+    const int row = 16 * t + (lane & 15), j = p * (kPair / F::kCols);
+    const Src s{raw + ((size_t)(row < rows_here ? row : 0) * nb + j) * F::kBlock, F::kBlock, row < rows_here ? nb - j : 0};
+    F::put(W + rec * F::kRec, s, lane);
 }
-constexpr int kRBK = 8, kPFK = 2, kNTK = 768;   // K-quants: the Q6_K structure
 
 } // namespace gs
 
 // ------------------------------------------------------------- host side ---
 struct gs_qmatrix {
     uint32_t qtype;
-    size_t rows, cols, nb;     // nb: blocks per row
+    size_t rows, cols;
+    int np, tiles;             // records per row tile, row tiles
     int device;
-    int cus;                   // compute units: one 1024-thread workgroup each on the register paths
-    uint8_t *base;             // one device allocation holding the planes
-    gs::Q6Planes q6;           // Q6_K
-    gs::KPlanes kq;            // Q4_K / Q5_K
-    gs::Q3Planes q3;           // Q3_K
-    gs::Q4Planes q4;           // Q4_0 / Q4_1
-    const uint8_t *q8;         // Q8_0: int8 quants
-    const uint16_t *d;         // f16 d per block (Q8_0, Q6_K)
+    int cus;
+    uint8_t *base;             // the records
 };
 
 namespace {
-// get_scale_min_k4 (src/tensor/dequant.rs:141-148): the 6-bit scale and min
-// of sub-block j from the block's 12 packed bytes.
-void scale_min_k4(int j, const uint8_t *q, uint8_t *d, uint8_t *m)
+
+// Calls f with a value of the format of `qtype`.
+template <class Fn> int with_format(uint32_t qtype, Fn f)
 {
-    if (j < 4) {
-        *d = q[j] & 63;
-        *m = q[j + 4] & 63;
-    } else {
-        *d = (uint8_t)((q[j + 4] & 0xF) | ((q[j - 4] >> 6) << 4));
-        *m = (uint8_t)((q[j + 4] >> 4) | ((q[j] >> 6) << 4));
+    switch (qtype) {
+    case GS_QTYPE_Q4_0: return f(gs::Q4Fmt<false>());
+    case GS_QTYPE_Q4_1: return f(gs::Q4Fmt<true>());
+    case GS_QTYPE_Q8_0: return f(gs::Q8Fmt());
+    case GS_QTYPE_Q3_K: return f(gs::Q3Fmt());
+    case GS_QTYPE_Q4_K: return f(gs::KFmt<false>());
+    case GS_QTYPE_Q5_K: return f(gs::KFmt<true>());
+    case GS_QTYPE_Q6_K: return f(gs::Q6Fmt());
+    default: return GS_ERR_UNSUPPORTED;
     }
 }
 
-// Q4_K (144-byte blocks) / Q5_K (176) to the K planes (see KPlanes).
-int upload_kquant(bool q5, const uint8_t *src, size_t rows, size_t nb, gs_qmatrix *m)
+constexpr size_t kStage = (size_t)64 << 20;     // raw blocks on the device at a time
+
+// The matrix's blocks, a group of row tiles at a time, through a staging
+// buffer on the device to records.
+template <class F> int upload(gs_qmatrix *m, const uint8_t *src)
 {
-    const size_t n = rows * nb, np = 4 * n;
-    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t off_h = al(np * 32), off_sm = off_h + (q5 ? al(np * 8) : 0), off_dd = off_sm + al(np * 4);
-    const size_t total = off_dd + n * 4;
-    uint8_t *h = new (std::nothrow) uint8_t[total];
-    if (!h) return GS_ERR_NOMEM;
-    const size_t bb = q5 ? 176 : 144;
-    for (size_t i = 0; i < n; i++) {
-        const uint8_t *b = src + i * bb;
-        const uint8_t *scales = b + 4, *qh = b + 16, *qs = b + (q5 ? 48 : 16);
-        for (int st = 0; st < 4; st++) {
-            const size_t e = 4 * i + st;
-            memcpy(h + e * 32, qs + 32 * st, 32);
-            uint8_t sc1, m1, sc2, m2;
-            scale_min_k4(2 * st, scales, &sc1, &m1);
-            scale_min_k4(2 * st + 1, scales, &sc2, &m2);
-            const uint32_t w = (uint32_t)sc1 | ((uint32_t)m1 << 8) | ((uint32_t)sc2 << 16) | ((uint32_t)m2 << 24);
-            memcpy(h + off_sm + e * 4, &w, 4);
-            if (q5) {
-                uint32_t ha = 0, hb = 0;
-                for (int l = 0; l < 32; l++) {
-                    ha |= (uint32_t)((qh[l] >> (2 * st)) & 1u) << l;
-                    hb |= (uint32_t)((qh[l] >> (2 * st + 1)) & 1u) << l;
-                }
-                memcpy(h + off_h + e * 8, &ha, 4);
-                memcpy(h + off_h + e * 8 + 4, &hb, 4);
-            }
-        }
-        memcpy(h + off_dd + i * 4, b, 4);   // d, dmin (f16 each)
-    }
-    if (hipMalloc((void **)&m->base, total) != hipSuccess) {
+    const size_t nb = m->cols / F::kCols, row_bytes = nb * F::kBlock;
+    const size_t step = kStage / (16 * row_bytes) > 0 ? kStage / (16 * row_bytes) : 1;
+    const size_t most = step < (size_t)m->tiles ? step : (size_t)m->tiles;
+    if (hipMalloc((void **)&m->base, (size_t)m->tiles * m->np * F::kRec) != hipSuccess) {
         (void)hipGetLastError();
-        delete[] h;
+        m->base = nullptr;
         return GS_ERR_NOMEM;
     }
-    const hipError_t ce = hipMemcpy(m->base, h, total, hipMemcpyHostToDevice);
-    delete[] h;
-    if (ce != hipSuccess) { (void)hipFree(m->base); m->base = nullptr; return GS_ERR_HIP; }
-    m->kq = gs::KPlanes{m->base, q5 ? (const uint2 *)(m->base + off_h) : nullptr,
-                        (const uint32_t *)(m->base + off_sm), (const uint32_t *)(m->base + off_dd)};
-    return GS_OK;
-}
-// Q4_0 (18-byte blocks) / Q4_1 (20) to the Q4 planes (see Q4Planes).
-int upload_q4(bool q41, const uint8_t *src, size_t rows, size_t nb, gs_qmatrix *m)
-{
-    const size_t n = rows * nb;
-    const size_t off_d = (n * 16 + 255) & ~(size_t)255;
-    const size_t total = off_d + n * (q41 ? 4 : 2);
-    uint8_t *h = new (std::nothrow) uint8_t[total];
-    if (!h) return GS_ERR_NOMEM;
-    const size_t bb = q41 ? 20 : 18;
-    for (size_t i = 0; i < n; i++) {
-        const uint8_t *b = src + i * bb;
-        memcpy(h + i * 16, b + (q41 ? 4 : 2), 16);
-        memcpy(h + off_d + i * (q41 ? 4 : 2), b, q41 ? 4 : 2);   // d (, m): f16 each
-    }
-    if (hipMalloc((void **)&m->base, total) != hipSuccess) {
+    uint8_t *raw = nullptr;
+    if (hipMalloc((void **)&raw, most * 16 * row_bytes) != hipSuccess) {
         (void)hipGetLastError();
-        delete[] h;
         return GS_ERR_NOMEM;
     }
-    const hipError_t ce = hipMemcpy(m->base, h, total, hipMemcpyHostToDevice);
-    delete[] h;
-    if (ce != hipSuccess) { (void)hipFree(m->base); m->base = nullptr; return GS_ERR_HIP; }
-    m->q4 = gs::Q4Planes{m->base, q41 ? nullptr : (const uint16_t *)(m->base + off_d),
-                         q41 ? (const uint32_t *)(m->base + off_d) : nullptr};
-    return GS_OK;
+    int rc = GS_OK;
+    for (size_t t = 0; t < (size_t)m->tiles && rc == GS_OK; t += step) {
+        const size_t n = (size_t)m->tiles - t < step ? (size_t)m->tiles - t : step;
+        const size_t rows = m->rows - 16 * t < 16 * n ? m->rows - 16 * t : 16 * n;
+        if (hipMemcpy(raw, src + 16 * t * row_bytes, rows * row_bytes, hipMemcpyHostToDevice) != hipSuccess) { rc = GS_ERR_HIP; break; }
+        const size_t threads = n * m->np * 64;
+        hipLaunchKernelGGL(gs::repack_kernel<F>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, nullptr, raw,
+                           m->base + t * m->np * F::kRec, (int)rows, (int)nb, m->np, (int)n);
+        if (hipGetLastError() != hipSuccess) rc = GS_ERR_HIP;
+    }
+    if (hipStreamSynchronize(nullptr) != hipSuccess) rc = GS_ERR_HIP;
+    (void)hipFree(raw);
+    return rc;
 }
 
-// The signed 6-bit scale of sub-block is of a Q3_K block in the GGUF
-// packing: low nibble from byte is % 8 (bits 0-3 for is < 8, 4-7 above),
-// top two bits from bits 2 (is / 4) of byte 8 + is % 4; minus 32.
-int q3k_scale(const uint8_t *sc, int is)
+template <class F, bool MULTI>
+int gemv(const gs_qmatrix *m, const float *x, float *out, int B, hipStream_t st)
 {
-    const int k = is >> 2, j = is & 3;
-    const uint8_t nb = sc[(k & 1) * 4 + j];
-    const int low = k < 2 ? (nb & 0xF) : (nb >> 4);
-    return (low | (((sc[8 + j] >> (2 * k)) & 3) << 4)) - 32;
+    const int nw = MULTI ? gs::kMaxWaves : m->np;
+    int blocks = m->cus * (gs::kMaxWaves / nw);         // 16 waves per CU
+    int tpb = (m->tiles + blocks - 1) / blocks;
+    tpb = (tpb + gs::kInFlight - 1) / gs::kInFlight * gs::kInFlight;
+    blocks = (m->tiles + tpb - 1) / tpb;
+    hipLaunchKernelGGL((gs::qgemv_kernel<F, MULTI>), dim3(blocks), dim3(64 * nw), gs::gemv_lds(nw), st, m->base, x, out,
+                       (int)m->rows, (int)m->cols, m->np, B, m->tiles, tpb);
+    return hipGetLastError() == hipSuccess ? GS_OK : GS_ERR_HIP;
 }
 
-// Q3_K (110-byte blocks) to the Q3 planes (see Q3Planes).
-int upload_q3k(const uint8_t *src, size_t rows, size_t nb, gs_qmatrix *m)
+template <class F, int VT, int RT>
+int gemm_rt(const gs_qmatrix *m, const float *x, float *out, int B, int per, int groups, int blocks, int tpb, hipStream_t st)
 {
-    const size_t n = rows * nb, np = 4 * n;
-    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t off_s = al(np * 32), off_d = off_s + al(np * 4);
-    const size_t total = off_d + n * 2;
-    uint8_t *h = new (std::nothrow) uint8_t[total];
-    if (!h) return GS_ERR_NOMEM;
-    for (size_t i = 0; i < n; i++) {
-        const uint8_t *b = src + i * 110;
-        const uint8_t *hm = b, *qs = b + 32, *sc = b + 96;
-        for (int qq = 0; qq < 4; qq++) {
-            const int nn = qq >> 1, l0 = (qq & 1) * 16;
-            const size_t e = 4 * i + qq;
-            for (int j = 0; j < 4; j++)
-                for (int k = 0; k < 16; k++) {
-                    const int l = l0 + k;
-                    const uint8_t u = (uint8_t)(((qs[32 * nn + l] >> (2 * j)) & 3u) | (((hm[l] >> (4 * nn + j)) & 1u) << 2));
-                    uint8_t &dst = h[e * 32 + 16 * (j >> 1) + k];
-                    dst = (j & 1) ? (uint8_t)(dst | (u << 4)) : u;
-                }
-            for (int j = 0; j < 4; j++)
-                h[off_s + e * 4 + j] = (uint8_t)(int8_t)q3k_scale(sc, 8 * nn + 2 * j + l0 / 16);
-        }
-        memcpy(h + off_d + i * 2, b + 108, 2);
-    }
-    if (hipMalloc((void **)&m->base, total) != hipSuccess) {
-        (void)hipGetLastError();
-        delete[] h;
-        return GS_ERR_NOMEM;
-    }
-    const hipError_t ce = hipMemcpy(m->base, h, total, hipMemcpyHostToDevice);
-    delete[] h;
-    if (ce != hipSuccess) { (void)hipFree(m->base); m->base = nullptr; return GS_ERR_HIP; }
-    m->q3 = gs::Q3Planes{m->base, (const uint32_t *)(m->base + off_s), (const uint16_t *)(m->base + off_d)};
-    return GS_OK;
+    hipLaunchKernelGGL((gs::qgemm_kernel<F, VT, RT>), dim3(blocks, groups), dim3(64 * gs::kGemmWaves), 0, st, m->base, x,
+                       out, (int)m->rows, (int)m->cols, m->np, B, per, m->tiles, tpb);
+    return hipGetLastError() == hipSuccess ? GS_OK : GS_ERR_HIP;
 }
+
+template <class F, int VT>
+int gemm(const gs_qmatrix *m, const float *x, float *out, int B, int per, int groups, hipStream_t st)
+{
+    int blocks = m->cus / groups;
+    if (blocks < 1) blocks = 1;
+    const int tpb = (m->tiles + blocks - 1) / blocks;
+    blocks = (m->tiles + tpb - 1) / tpb;
+    // rounds of at most 5 tiles per wave, as even as they can be
+    const int rounds = (tpb + 5 * gs::kGemmWaves - 1) / (5 * gs::kGemmWaves);
+    const int rt = ((tpb + rounds - 1) / rounds + gs::kGemmWaves - 1) / gs::kGemmWaves;
+    switch (rt) {
+    case 1: return gemm_rt<F, VT, 1>(m, x, out, B, per, groups, blocks, tpb, st);
+    case 2: return gemm_rt<F, VT, 2>(m, x, out, B, per, groups, blocks, tpb, st);
+    case 3: return gemm_rt<F, VT, 3>(m, x, out, B, per, groups, blocks, tpb, st);
+    case 4: return gemm_rt<F, VT, 4>(m, x, out, B, per, groups, blocks, tpb, st);
+    default: return gemm_rt<F, VT, 5>(m, x, out, B, per, groups, blocks, tpb, st);
+    }
+}
+
+template <class F>
+int project(const gs_qmatrix *m, const float *x, float *out, int B, hipStream_t st)
+{
+    if (B <= gs::kVecs)
+        return m->np <= gs::kMaxWaves ? gemv<F, false>(m, x, out, B, st) : gemv<F, true>(m, x, out, B, st);
+    const int groups = (B + 31) / 32, per = (B + groups - 1) / groups;
+    return per <= 16 ? gemm<F, 1>(m, x, out, B, per, groups, st) : gemm<F, 2>(m, x, out, B, per, groups, st);
+}
+
 } // namespace
 
 extern "C" {
@@ -964,82 +1041,25 @@ int gs_qmatrix_upload(uint32_t qtype, const void *blocks, size_t rows, size_t co
     if (!out) return GS_ERR_INVALID;
     *out = nullptr;
     if (!blocks || rows == 0 || cols == 0) return GS_ERR_INVALID;
-    if (qtype != GS_QTYPE_Q8_0 && qtype != GS_QTYPE_Q6_K && qtype != GS_QTYPE_Q4_K && qtype != GS_QTYPE_Q5_K &&
-        qtype != GS_QTYPE_Q4_0 && qtype != GS_QTYPE_Q4_1 && qtype != GS_QTYPE_Q3_K)
-        return GS_ERR_UNSUPPORTED;
-    if (qtype == GS_QTYPE_Q4_K || qtype == GS_QTYPE_Q5_K || qtype == GS_QTYPE_Q4_0 || qtype == GS_QTYPE_Q4_1 ||
-        qtype == GS_QTYPE_Q3_K) {
-        const bool q4 = qtype == GS_QTYPE_Q4_0 || qtype == GS_QTYPE_Q4_1;
-        const size_t bw = q4 ? 32 : 256;
-        if (cols % bw != 0 || cols > (size_t)gs::kMaxCols || rows > 0x7fffffffu) return GS_ERR_UNSUPPORTED;
-        // 32-bit byte offsets of the widest plane
-        if (rows * (cols / 64) >= (q4 ? (1ull << 29) : (1ull << 27))) return GS_ERR_UNSUPPORTED;
-        gs_qmatrix *m = new (std::nothrow) gs_qmatrix();
-        if (!m) return GS_ERR_NOMEM;
-        m->qtype = qtype; m->rows = rows; m->cols = cols; m->nb = cols / bw;
-        if (hipGetDevice(&m->device) != hipSuccess ||
-            hipDeviceGetAttribute(&m->cus, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess) {
-            delete m; return GS_ERR_HIP;
-        }
-        if (m->cus <= 0) m->cus = 256;
-        const int rc = q4 ? upload_q4(qtype == GS_QTYPE_Q4_1, (const uint8_t *)blocks, rows, cols / 32, m)
-                       : qtype == GS_QTYPE_Q3_K ? upload_q3k((const uint8_t *)blocks, rows, cols / 256, m)
-                       : upload_kquant(qtype == GS_QTYPE_Q5_K, (const uint8_t *)blocks, rows, cols / 256, m);
-        if (rc != GS_OK) { delete m; return rc; }
-        *out = m;
-        return GS_OK;
-    }
-    const bool q6 = qtype == GS_QTYPE_Q6_K;
-    const size_t bw = q6 ? 256 : 32;        // weights per block
-    const size_t bb = q6 ? 210 : 34;        // bytes per GGUF block
+    size_t bw = 0;
+    if (int rc = with_format(qtype, [&](auto f) { bw = decltype(f)::kCols; return GS_OK; })) return rc;
     if (cols % bw != 0 || cols > (size_t)gs::kMaxCols || rows > 0x7fffffffu) return GS_ERR_UNSUPPORTED;
-    if (rows * (cols / 64) >= (1ull << 28)) return GS_ERR_UNSUPPORTED;   // 32-bit chunk offsets
-    const size_t nb = cols / bw, n = rows * nb;
-    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    // planes: Q6_K a | b | c (64 bytes per block each) | scale words (16) | d (2);
-    //         Q8_0 quants (32 bytes per block) | d (2)
-    const size_t pa = q6 ? al(n * 64) : al(n * 32);
-    const size_t off_b = pa, off_c = q6 ? 2 * pa : pa, off_s = q6 ? 3 * pa : pa;
-    const size_t off_d = q6 ? off_s + al(n * 16) : pa;
-    const size_t total = off_d + n * 2;
-    uint8_t *h = new (std::nothrow) uint8_t[total];
-    if (!h) return GS_ERR_NOMEM;
-    const uint8_t *src = (const uint8_t *)blocks;
-    for (size_t i = 0; i < n; i++) {
-        const uint8_t *b = src + i * bb;
-        if (q6) {
-            // quarter qq = 2h + l0/16 of block i: element e = 4i + qq of each plane
-            for (int qq = 0; qq < 4; qq++) {
-                const int hh = qq >> 1, l0 = (qq & 1) * 16, is = l0 / 16;
-                const size_t e = 4 * i + qq;
-                memcpy(h + e * 16, b + 64 * hh + l0, 16);                  // ql[64h + l0 ..]
-                memcpy(h + off_b + e * 16, b + 64 * hh + 32 + l0, 16);     // ql[64h + 32 + l0 ..]
-                memcpy(h + off_c + e * 16, b + 128 + 32 * hh + l0, 16);    // qh[32h + l0 ..]
-                for (int g = 0; g < 4; g++) h[off_s + e * 4 + g] = b[192 + 8 * hh + is + 2 * g];
-            }
-            memcpy(h + off_d + i * 2, b + 208, 2);
-        } else {
-            memcpy(h + i * 32, b + 2, 32);
-            memcpy(h + off_d + i * 2, b, 2);
-        }
-    }
+    // the size limits of each type's matrices
+    const bool q4 = qtype == GS_QTYPE_Q4_0 || qtype == GS_QTYPE_Q4_1;
+    const bool q68 = qtype == GS_QTYPE_Q6_K || qtype == GS_QTYPE_Q8_0;
+    if (rows * (cols / 64) >= (q4 ? 1ull << 29 : q68 ? 1ull << 28 : 1ull << 27)) return GS_ERR_UNSUPPORTED;
     gs_qmatrix *m = new (std::nothrow) gs_qmatrix();
-    if (!m) { delete[] h; return GS_ERR_NOMEM; }
-    m->qtype = qtype; m->rows = rows; m->cols = cols; m->nb = nb;
+    if (!m) return GS_ERR_NOMEM;
+    m->qtype = qtype; m->rows = rows; m->cols = cols;
+    m->np = (int)((cols + gs::kPair - 1) / gs::kPair);
+    m->tiles = (int)((rows + 15) / 16);
     if (hipGetDevice(&m->device) != hipSuccess ||
         hipDeviceGetAttribute(&m->cus, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess) {
-        delete[] h; delete m; return GS_ERR_HIP;
+        delete m; return GS_ERR_HIP;
     }
     if (m->cus <= 0) m->cus = 256;
-    if (hipMalloc((void **)&m->base, total) != hipSuccess) {
-        (void)hipGetLastError(); delete[] h; delete m; return GS_ERR_NOMEM;
-    }
-    const hipError_t ce = hipMemcpy(m->base, h, total, hipMemcpyHostToDevice);
-    delete[] h;
-    if (ce != hipSuccess) { (void)hipFree(m->base); delete m; return GS_ERR_HIP; }
-    m->d = (const uint16_t *)(m->base + off_d);
-    if (q6) m->q6 = gs::Q6Planes{m->base, m->base + off_b, m->base + off_c, (const uint32_t *)(m->base + off_s), m->d};
-    else m->q8 = m->base;
+    const int rc = with_format(qtype, [&](auto f) { return upload<decltype(f)>(m, (const uint8_t *)blocks); });
+    if (rc != GS_OK) { if (m->base) (void)hipFree(m->base); delete m; return rc; }
     *out = m;
     return GS_OK;
 }
@@ -1070,46 +1090,13 @@ int gs_gemv(const gs_qmatrix *m, const float *d_x, size_t B, float *d_out, void 
 {
     if (!m || (B > 0 && (!d_x || !d_out))) return GS_ERR_INVALID;
     if (((uintptr_t)d_x & 15u) != 0 || (B > 1 && (m->cols & 3) != 0)) return GS_ERR_INVALID;   // x is read as float4
-    const hipStream_t st = (hipStream_t)stream;
-    const int rows = (int)m->rows, nb = (int)m->nb;
-    for (size_t b = 0; b < B; b++) {
-        const float *x = d_x + b * m->cols;
-        float *o = d_out + b * m->rows;
-        if (m->qtype == GS_QTYPE_Q4_K || m->qtype == GS_QTYPE_Q5_K) {
-            const bool q5 = m->qtype == GS_QTYPE_Q5_K;
-            if (4 * nb <= 64) {
-                if (q5) hipLaunchKernelGGL((gs::kq_gemv_xreg<true, gs::kRBK, gs::kPFK, gs::kNTK>), dim3(m->cus), dim3(gs::kNTK), 0, st, m->kq, x, o, rows, nb);
-                else hipLaunchKernelGGL((gs::kq_gemv_xreg<false, gs::kRBK, gs::kPFK, gs::kNTK>), dim3(m->cus), dim3(gs::kNTK), 0, st, m->kq, x, o, rows, nb);
-            } else {
-                if (q5) hipLaunchKernelGGL(gs::kq_gemv_lds<true>, dim3(2 * m->cus), dim3(gs::kGemvThreads), 0, st, m->kq, x, o, rows, nb);
-                else hipLaunchKernelGGL(gs::kq_gemv_lds<false>, dim3(2 * m->cus), dim3(gs::kGemvThreads), 0, st, m->kq, x, o, rows, nb);
-            }
-        } else if (m->qtype == GS_QTYPE_Q4_0 || m->qtype == GS_QTYPE_Q4_1) {
-            const bool q41 = m->qtype == GS_QTYPE_Q4_1;
-            if (nb <= 64 * gs::kQ4Blocks) {
-                if (q41) hipLaunchKernelGGL((gs::q4_gemv_xreg<true, gs::kRB4, gs::kPF4, gs::kNT4>), dim3(m->cus), dim3(gs::kNT4), 0, st, m->q4, x, o, rows, nb);
-                else hipLaunchKernelGGL((gs::q4_gemv_xreg<false, gs::kRB4, gs::kPF4, gs::kNT4>), dim3(m->cus), dim3(gs::kNT4), 0, st, m->q4, x, o, rows, nb);
-            } else {
-                if (q41) hipLaunchKernelGGL(gs::q4_gemv_lds<true>, dim3(2 * m->cus), dim3(gs::kGemvThreads), 0, st, m->q4, x, o, rows, nb);
-                else hipLaunchKernelGGL(gs::q4_gemv_lds<false>, dim3(2 * m->cus), dim3(gs::kGemvThreads), 0, st, m->q4, x, o, rows, nb);
-            }
-        } else if (m->qtype == GS_QTYPE_Q3_K) {
-            if (4 * nb <= 64)
-                hipLaunchKernelGGL((gs::q3k_gemv_xreg<gs::kRB3, gs::kPF3, gs::kNT3>), dim3(m->cus), dim3(gs::kNT3), 0, st, m->q3, x, o, rows, nb);
-            else
-                hipLaunchKernelGGL(gs::q3k_gemv_lds, dim3(2 * m->cus), dim3(gs::kGemvThreads), 0, st, m->q3, x, o, rows, nb);
-        } else if (m->qtype == GS_QTYPE_Q6_K) {
-            if (4 * nb <= 64)
-                hipLaunchKernelGGL((gs::q6k_gemv_xreg<gs::kRB6, gs::kPF6, gs::kNT6>), dim3(m->cus), dim3(gs::kNT6), 0, st, m->q6, x, o, rows, nb);
-            else
-                hipLaunchKernelGGL(gs::q6k_gemv_lds, dim3(2 * m->cus), dim3(gs::kGemvThreads), 0, st, m->q6, x, o, rows, nb);
-        } else {
-            if (2 * nb <= 64 * gs::kQ8Halves)
-                hipLaunchKernelGGL((gs::q80_gemv_xreg<gs::kRB8, gs::kPF8, gs::kNT8>), dim3(m->cus), dim3(gs::kNT8), 0, st, m->q8, m->d, x, o, rows, nb);
-            else
-                hipLaunchKernelGGL(gs::q80_gemv_lds, dim3(2 * m->cus), dim3(gs::kGemvThreads), 0, st, m->q8, m->d, x, o, rows, nb);
-        }
-        if (hipGetLastError() != hipSuccess) return GS_ERR_HIP;
+    // up to 16384 vectors per launch (groups of 16 along the grid's y)
+    for (size_t b = 0; b < B; b += 16384) {
+        const int n = (int)(B - b < 16384 ? B - b : 16384);
+        const int rc = with_format(m->qtype, [&](auto f) {
+            return project<decltype(f)>(m, d_x + b * m->cols, d_out + b * m->rows, n, (hipStream_t)stream);
+        });
+        if (rc != GS_OK) return rc;
     }
     return GS_OK;
 }

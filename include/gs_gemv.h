@@ -70,8 +70,10 @@ typedef struct gs_qmatrix gs_qmatrix;
 /* Replaces Gpu::upload (src/gpu/mod.rs:222-238) for the seven block types above.
  * `blocks` is a host pointer to rows*cols weights in GGUF block order
  * (row-major, dims[0] = cols as in QuantTensor::new, src/tensor/dequant.rs:256-263).
- * The blocks are split into the device layout (bit planes, int8 scales, f16 d)
- * and copied to the current HIP device; synchronous.  cols must be a multiple
+ * The blocks are copied to the current HIP device, through a staging buffer of
+ * up to 64 MB, and rearranged there (records of 16 rows x 256 columns in the
+ * order the kernels read them; rows of the matrix are padded to 16 and columns
+ * to 256); synchronous.  cols must be a multiple
  * of the block size (32 / 256) -- where the reference's upload returns None
  * and falls back to the CPU, this returns GS_ERR_UNSUPPORTED (for Q4_0 and Q4_1
  * the reference has no such check and would read misaligned blocks) -- and at
@@ -84,10 +86,11 @@ int gs_qmatrix_shape(const gs_qmatrix *m, uint32_t *qtype, size_t *rows, size_t 
 /* Replaces Gpu::cmd_gemv (src/gpu/mod.rs:438-443): for b < B,
  * d_out[b*rows + r] = sum_c W[r][c] * d_x[b*cols + c].  Device pointers;
  * asynchronous on `stream` (NULL = default stream).  B = 1 is the reference's
- * decode step; each further vector is another full pass over the weights (a
- * GEMV per vector, not a GEMM), so this entry is meant for small B: a
- * batch of hundreds of vectors should bring its own GEMM and hand the logits
- * to the sampler. */
+ * decode step; up to 32 vectors share one pass over the weights (the matrix
+ * cores take them together; x is split into two f16 parts whose products are
+ * added in f32, with an error no larger than that of f32 arithmetic), larger
+ * B goes in groups of up to 32.  An infinity or NaN in a vector makes its own
+ * logits non-finite and no other vector's. */
 int gs_gemv(const gs_qmatrix *m, const float *d_x, size_t B, float *d_out, void *stream);
 
 #ifdef __cplusplus

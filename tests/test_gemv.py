@@ -446,3 +446,69 @@ def test_gemv_full_lm_head(gpu, torch, oracle, qt, rows, cols):
     """Full output-projection shapes, every row against the oracle."""
     print("gemv full", qt, rows, cols, flush=True)
     _gpu_check(gpu, torch, oracle, qt, rows, cols, seed=rows % 1000 + qt)
+
+
+# ---- several vectors per call ---------------------------------------------------
+ALL_TYPES = (Q4_0, Q4_1, Q8_0, Q3_K, Q4_K, Q5_K, Q6_K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", ALL_TYPES)
+@pytest.mark.parametrize("rows,cols,B", [
+    (1, 256, 4), (33, 768, 2),          # up to 4 vectors: one kernel; rows of a part of a tile
+    (15, 256, 5), (17, 512, 16),        # up to 16: one tile of vectors, odd and even record counts
+    (257, 1280, 17), (129, 2048, 32),   # up to 32: two tiles
+    (64, 4352, 3), (64, 4352, 9),       # more columns than one block's waves hold (17 records)
+    (50, 512, 33), (50, 512, 70),       # more than 32: groups of vectors
+])
+def test_gemv_vectors(gpu, torch, oracle, qt, rows, cols, B):
+    """Every vector of a call, at the edges of the row tiles, the records and
+    the vector tiles."""
+    print("gemv vectors", qt, rows, cols, B, flush=True)
+    _gpu_check(gpu, torch, oracle, qt, rows, cols, seed=rows + cols + B, B=B, x_kind="spiky")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt,cols", [(Q4_0, 32), (Q4_0, 288), (Q4_1, 96), (Q8_0, 480), (Q8_0, 2016)])
+@pytest.mark.parametrize("B", [1, 7, 20])
+def test_gemv_ragged_columns(gpu, torch, oracle, qt, cols, B):
+    """Rows whose columns end inside a record of 256."""
+    print("gemv ragged", qt, cols, B, flush=True)
+    _gpu_check(gpu, torch, oracle, qt, 100, cols, seed=cols + B, B=B)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [32769, 70001, 100003, 131073, 165001])
+def test_gemv_tiles_per_wave(gpu, torch, oracle, rows):
+    """One to five row tiles per wave, and two rounds of them (256 CUs)."""
+    for qt, B in ((Q4_K, 5), (Q6_K, 18)):
+        print("gemv tiles", qt, rows, B, flush=True)
+        _gpu_check(gpu, torch, oracle, qt, rows, 256, seed=rows % 1000, B=B)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [3, 12])
+def test_gemv_wide_and_nonfinite(gpu, torch, oracle, B):
+    """x over a factor of 2^40 in one vector, and vectors with infinities and
+    NaNs beside it: each vector's result is its own."""
+    import workloads
+    rng = np.random.default_rng(B)
+    rows, cols = 100, 1024
+    x = rng.standard_normal((B, cols)).astype(np.float32)
+    x[0] *= np.exp2(rng.uniform(-20, 20, cols)).astype(np.float32)
+    x[1, 5] = np.inf
+    x[2, 700] = np.nan
+    for qt in ALL_TYPES:
+        blocks = workloads.synth_qblocks(qt, rows, cols, seed=B)
+        m = gpu.QMatrix(qt, blocks, rows, cols)
+        d_o = torch.zeros((B, rows), device="cuda")
+        m.gemv(torch.from_numpy(x).cuda(), d_o, B=B)
+        got = d_o.cpu().numpy()
+        m.close()
+        assert not np.isfinite(got[1]).any() and np.isnan(got[2]).all(), qt
+        for b in [b for b in range(B) if b not in (1, 2)]:
+            w = np.abs(oracle.dequant(qt, blocks, rows * cols).astype(np.float64)).max()
+            ex, ab = oracle.matvec(qt, blocks, rows, cols, x[b], nthreads=4, exact=True)
+            # the parts of x: 2^-22 of each value, 2^-39 of the largest; 32-bit sums
+            tol = 2.0 ** -16 * ab + w * 2.0 ** -22 * np.abs(x[b]).astype(np.float64).sum() * 64
+            assert (np.abs(got[b] - ex) <= tol).all(), (qt, b)
