@@ -38,7 +38,7 @@
 // the row then takes the sort-based path (the same result, slower).
 
 // Failure exits (development builds record the line per row).
-#if defined(GS_TIMING) || defined(GS_DIAG)
+#if defined(GS_TIMING) || defined(GS_ROWDIAG)
 // per row (< 1024): [0] failing line of the row, [1] failing line of a walk,
 // [2..7] statistics (see F_STAT uses)
 __device__ int g_vdiag[1024 * 16];
@@ -1262,7 +1262,7 @@ __device__ bool full_v2_row(RowSmem &sm, const float *row, int V, float T, float
             pre = f_block_excl_f64_buf(loc, &tot, round == 0 ? sm.red_f64 : sm.red_f64b) + osum;   // (buffers alternate)
         }
         __syncthreads();
-#if defined(GS_TIMING) || defined(GS_DIAG)
+#if defined(GS_TIMING) || defined(GS_ROWDIAG)
         if (t == 0 && blockIdx.x < 1024) g_vdiag[blockIdx.x * 16 + 14] = __float_as_int((float)(tot + osum));
 #endif
         F_TS(2);

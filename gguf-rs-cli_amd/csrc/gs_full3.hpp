@@ -34,7 +34,7 @@
 
 // Development builds record per row (< 1024) the failing line ([0]) and
 // statistics, and per row (< 256) stage timestamps.
-#if defined(GS_TIMING) || defined(GS_DIAG)
+#if defined(GS_TIMING) || defined(GS_ROWDIAG)
 __device__ int g_v3diag[1024 * 32];
 __device__ uint32_t g_v3t[256 * 32];
 #define F3_STAT(k, v) do { if (threadIdx.x == 0 && blockIdx.x < 1024) g_v3diag[blockIdx.x * 32 + (k)] = (int)(v); } while (0)

@@ -1691,7 +1691,7 @@ extern "C" int gs_debug_fails(int *out)
     return hipMemcpyFromSymbol(out, HIP_SYMBOL(gs::g_fails), sizeof(int) * 1280) == hipSuccess ? 0 : -5;
 }
 #endif
-#if defined(GS_TIMING) || defined(GS_DIAG)
+#if defined(GS_TIMING) || defined(GS_ROWDIAG)
 extern "C" int gs_debug_v3dump(int *out)
 {
     return hipMemcpyFromSymbol(out, HIP_SYMBOL(gs::g_v3dump), sizeof(int) * 64 * 256) == hipSuccess ? 0 : -5;
