@@ -894,7 +894,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
 
     // ---- pass 1 (HBM): counts, masses of the top bins, max, NaN -------------
     // Bins are of t = cb - y / w, cb = (m0 + 3) / w, m0 the maximum of the
-    // first round of loads: bin b = floor(t) in [0, kFBins); t < 0 (elements
+    // first round of loads (of ids that are not penalized): bin b = floor(t) in [0, kFBins); t < 0 (elements
     // more than 3 above m0) go to the overflow list, t >= kFBins (more than
     // 18.5 below) add 0 to every sum.
     float tmax = -INFINITY;
@@ -930,10 +930,27 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
                 for (int u = 0; u < kUnroll; u++) nv[u] = ldg(r4 + min(base + kThreads * kUnroll + u * kThreads + t, n4 - 1));
             }
             if (base == 0) {
-                float lm = -INFINITY;
+                // (without the penalized ids: a row whose largest raw value is
+                // penalized would have its maximum below m0)
+                float lm;
+                for (uint32_t gone = 0u;;) {
+                    lm = -INFINITY;
+                    int at = 0;
 #pragma unroll
-                for (int u = 0; u < kUnroll; u++)
-                    if (u * kThreads + t < n4) lm = fmaxf(lm, fmaxf(fmaxf(v[u].x, v[u].y), fmaxf(v[u].z, v[u].w)));
+                    for (int u = 0; u < kUnroll; u++) {
+                        const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                        for (int c = 0; c < 4; c++)
+                            if (u * kThreads + t < n4 && e[c] > lm && !((gone >> (4 * u + c)) & 1u)) {
+                                lm = e[c];
+                                at = 4 * u + c;
+                            }
+                    }
+                    if (!has_pen || lm == -INFINITY ||
+                        hash_find(sm, (uint32_t)(h0 + 4 * ((at >> 2) * kThreads + t) + (at & 3))) < 0)
+                        break;
+                    gone |= 1u << at;
+                }
                 m0 = ydiv(f_block_max(lm, sm));
                 if (!isfinite(m0)) return false;
                 cb = (float)(((double)m0 + (double)kFDUp) * (double)kFInvW);
@@ -980,7 +997,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
     // segments must hold room for them) -------------------------------------
     if (has_pen) {
         for (int j = t; j < f.nover; j += kThreads)
-            if (hash_find(sm, f_entry_id(f.over[j])) >= 0) f.over[j] = 0ull;
+            if (hash_find(sm, f_entry_id(f.over[j])) >= 0) f.over[j] = f3_dead(f.over[j]);   // (unique: the sort ranks it)
         __syncthreads();
         for (int s = t; s < kHashSlots; s += kThreads) {
             const uint32_t id = sm.hkey[s];
@@ -1023,7 +1040,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
         double osum = 0.0;
         for (int j = t; j < nover; j += kThreads) {
             const uint64_t en = f.over[j];
-            if (en) osum += (double)glibc_expf_tab(f_entry_y(en) - m, f.exptab);
+            if (f3_live(en)) osum += (double)glibc_expf_tab(f_entry_y(en) - m, f.exptab);
         }
         double otot;
         f_block_excl_f64_buf(osum, &otot, sm.red_f64);
@@ -1084,7 +1101,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
 
     // ---- seq-1 roles: windows (the sum may change binade in the bin), the
     // level range of every other bin, and the head: the smallest bH whose
-    // runs' levels below fit kF3L1 ------------------------------------------
+    // runs' levels below fit the budget ------------------------------------------
     int bmax = -1;    // the bin of the maximum (the head holds it)
     {
         const int im = f3_tidx(m, cb);
@@ -1095,8 +1112,11 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
 #pragma unroll
         for (int q = 0; q < kPer; q++) {
             const int b = kPer * t + q;
-            const double lo = (double)f.pre[b], hi = (double)f.pre[b + 1];
-            const bool win = !(lo > 0.0) || f_dexp(lo * dl) != f_dexp(hi * dh);
+            // (the maximum's own summand is 1: the sum is at least 1 after
+            // it, however little the rest of the row adds)
+            const double least = b > bmax ? 1.0 : 0.0;
+            const double lo = fmax((double)f.pre[b], least), hi = (double)f.pre[b + 1];
+            const bool win = !(lo > 0.0) || f_dexp(fmax(lo * dl, least)) != f_dexp(hi * dh);
             const int e = lo > 0.0 ? f_dexp(lo) : 0;
             key[q] = win ? kF3KeyListed : (uint32_t)(e + 256);
             klo[q] = 1u;
@@ -1133,13 +1153,19 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
             ssum += c[q];
         }
         F3_TS(26);
+        // Budget of seq-1 levels: kF3L1, and few enough for seq 2, whose last
+        // grid is finer by up to 2 2^e / S (2^e the power of two below S:
+        // its sums end in [1/2, 1)), to fit kF3L23 below the same head.
+        const double P = (double)f.pre[kFBins];
+        const double finer = ldexp(2.0, f_dexp(P)) / P;
+        const uint32_t budget = (uint32_t)fmin((double)kF3L1, (double)(kF3L23 - 64) * (1.0 - 1.0 / 512.0) / finer);
         uint32_t call;
         const uint32_t sp = block_excl_u32(ssum, &call, sm);
         uint32_t run_pre = sp, cand = kFBins;
 #pragma unroll
         for (int q = 0; q < kPer; q++) {
             const int b = kPer * t + q;
-            if (cand == (uint32_t)kFBins && b > bmax && b >= 1 && call - run_pre <= (uint32_t)kF3L1) cand = (uint32_t)b;
+            if (cand == (uint32_t)kFBins && b > bmax && b >= 1 && call - run_pre <= budget) cand = (uint32_t)b;
             run_pre += c[q];
         }
         const int bH = f3_block_min(f, cand);
