@@ -69,6 +69,7 @@ constexpr uint32_t kF3KeyListed = 0xffffffffu, kF3KeyNone = 0xfffffffeu;
 // (the product's rounding, the constant's and v_exp_f32's 1 ulp); beyond,
 // every scaled summand is far below 1/2.  The bands hold that error, and for
 // seqs 2 and 3 the roundings of 1/S, of the products and of p and q.
+constexpr double kF3Cut = 1.0 / 32768.0;          // margin of a cut near the end of the row (plan B)
 constexpr float kF3Band1 = 7.62939453125e-6f;      // 2^-17
 constexpr float kF3Band23 = 1.52587890625e-5f;     // 2^-16
 constexpr double kF3Lo = 1.0 - 1.0 / 65536.0, kF3Hi = 1.0 + 1.0 / 65536.0;   // level range margins (2^-16)
@@ -1357,26 +1358,77 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
     // ---- plan B (seqs 2, 3): predicted sums from the seq-1 prediction
     // normalised by its total; the cut and the draw windows; runs ----------
     float cS = 0.0f, cS3lo = 0.0f, band3 = 0.0f;
+    bool cutting;       // the nucleus ends before the row does
     {
-        const double iP = 1.0 / (double)f.pre[kFBins];
         const double iS = 1.0 / (double)S;
         const double tp = (double)top_p, rd = (double)r;
-        if (nuc && tp * dh >= 1.0) F3_FAIL();           // the cut may not happen
-        if (!nuc && rd >= dl) F3_FAIL();                 // the draw may not happen
+        // A cut near the end of the row: seq 2 drops the summands below half
+        // a step of its own grid, so its total is not seq 1's over S (up to
+        // 1e-3 off), and the cut may not happen at all (every candidate is
+        // kept, s2 is the total).  There the sums are predicted again, from
+        // the mean rounded increments at seq 2's grids and, past the bins of
+        // known mass, with the error of seq 1's prediction (S is exact now,
+        // and that error comes from the bins next to those): good to a few
+        // 1e-6 in the tail, so the cut's margin is kF3Cut.  Below 0.98 the
+        // difference is far below the common margin.  A row that fails here
+        // is sorted whole (3.5 ms at V 256000): batches of 512 such rows with
+        // one at top_p 0.9993..0.9998 took 2656..3541 us, now 511..558.  Of
+        // 576 rows at top_p 0.98..0.99997 (V 3001..152064), 72 fail at
+        // 2^-15; 102 do at 2^-14 (more of them have no sure cut).
+        double iP = 1.0 / (double)f.pre[kFBins], end2 = 1.0, cl = dl, ch = dh;
+        if (nuc && tp >= 0.98) {
+            double ct[kPer], loc = 0.0;
+            const double base = (double)f.pre[0], shift = (double)S - (double)f.pre[kFBins];
+#pragma unroll
+            for (int q = 0; q < kPer; q++) {
+                const int b = kPer * t + q;
+                const double lo = (double)f.pre[b] * iP;
+                ct[q] = (double)f.pre[b + 1] - (double)f.pre[b];
+                if (b >= kFMassBins && f.cnt[b] && lo > 0.0) {
+                    const int ge = f_dexp(lo) - 23;
+                    const double uh = ldexp(e_at((double)b) * iS, -ge), ul = ldexp(e_at((double)(b + 1)) * iS, -ge);
+                    const double sh = uh - rint(uh), sl = ul - rint(ul);
+                    const double mean = uh > ul ? 0.5 * (uh + ul) - 0.5 * (sh * sh - sl * sl) / (uh - ul) : rint(uh);
+                    ct[q] = (double)f.cnt[b] * ldexp(mean, ge) * (double)S;
+                }
+                loc += ct[q];
+            }
+            double tot;
+            double lo = f_block_excl_f64_buf(loc, &tot, sm.red_f64) + base;     // (its barriers: pre read)
+#pragma unroll
+            for (int q = 0; q < kPer; q++) {
+                const int b = kPer * t + q;
+                f.pre[b] = (float)(b >= kFMassBins ? lo + shift : lo);
+                lo += ct[q];
+            }
+            if (t == kThreads - 1) f.pre[kFBins] = (float)(lo + shift);
+            __syncthreads();
+            iP = iS;
+            end2 = (double)f.pre[kFBins] * iS;
+            cl = 1.0 - kF3Cut;
+            ch = 1.0 + kF3Cut;
+        }
+        cutting = nuc && !(end2 * ch < tp);
+        if (cutting && tp * ch >= end2) F3_FAIL();      // the cut may or may not happen
+        if (!cutting && rd >= dl) F3_FAIL();             // the draw may not happen
         // s2 lies in [top_p, top_p + the cut element's summand + a rounding
         // step]: the summand is at most the first cut-window bin's largest
         // (or 1/S if the cut may lie in the head)
         uint32_t cand = kFBins;
-        if (nuc) {
+        if (cutting) {
 #pragma unroll
             for (int q = 0; q < kPer; q++) {
                 const int b = kPer * t + q;
-                if (cand == (uint32_t)kFBins && b >= bH && (double)f.pre[b + 1] * iP * dh >= tp) cand = (uint32_t)b;
+                if (cand == (uint32_t)kFBins && b >= bH && (double)f.pre[b + 1] * iP * ch >= tp) cand = (uint32_t)b;
             }
         }
         const int bcut = f3_block_min(f, cand);     // the first bin the cut may lie in
         double s2lo = 1.0, s2hi = 1.0;
-        if (nuc) {
+        if (nuc && !cutting) {
+            s2lo = (double)__double2float_rd(end2 * cl);
+            s2hi = (double)__double2float_ru(end2 * ch);
+        }
+        if (cutting) {
             const int bc = bcut;
             double vmax = iS;
             if (bc > bH && bc < kFBins) {
@@ -1405,9 +1457,9 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
             ku2[q] = ku3[q] = kF3NoU;
             rl[q] = 0u;
             if (b < bH) continue;
-            const bool past = nuc && lo2 * dl >= tp;
+            const bool past = cutting && lo2 * cl >= tp;
             if (past) continue;
-            const bool cw = nuc && hi2 * dh >= tp;
+            const bool cw = cutting && hi2 * ch >= tp;
             float ylo, yhi;
             f3_range(cb, b, &ylo, &yhi);
             const double pl = (double)f3_exp(ylo - m) * iS;
@@ -1689,13 +1741,13 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
         __syncthreads();
         F3_STAT(14, f.walk_res);
         F3_STAT(15, f.nreg);
-        if (f.walk_res != 1) F3_FAIL();
+        if (f.walk_res != (cutting ? 1 : 0)) F3_FAIL();
         s2 = f.s2;
         cut_arr = f.cut_arr;
         cut_pos = f.cut_pos;
         // the cut must not lie inside a run of seq 3 (walk 3 stops there)
-        if (cut_arr == 1u ? cut_pos >= nl3 : cut_pos >= headend) F3_FAIL();
-        if (cut_arr == 1u) {
+        if (cutting && (cut_arr == 1u ? cut_pos >= nl3 : cut_pos >= headend)) F3_FAIL();
+        if (cutting && cut_arr == 1u) {
             const uint64_t en = ldg(se3 + cut_pos);
             if (ldg(role + f3_bin(f_entry_y(en), cb)) & kF3In3) F3_FAIL();
         }
@@ -1739,7 +1791,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
         if (wave_id() == 0) {
             float c;
             uint32_t arr = 0u, pos = 0u;
-            const int res = f3_walk(f, stg_lds, headend, 1, segst, cend3, F3Above{r}, nuc,
+            const int res = f3_walk(f, stg_lds, headend, 1, segst, cend3, F3Above{r}, cutting,
                                     cut_arr, cut_pos, &c, &arr, &pos);
             if (lane_id() == 0) {
                 f.walk_res = res;

@@ -1,6 +1,7 @@
 """Full-vocabulary rows at the edges of the plans: rows whose largest logits
 are penalized, rows whose softmax sum lies a little above a power of two (the
-normalized sums then need the finest grids), and rows that the top logit
+normalized sums then need the finest grids; half of them with a nucleus that
+ends at the end of the row or not at all), and rows that the top logit
 dominates.  Tokens must equal the oracle's, and the rows must stay on the
 increment-histogram path (a fallback is exact too, but several times slower).
 """
@@ -33,6 +34,8 @@ def _case(shape, V, rng):
             y[i] = -np.inf
             R = np.log(np.exp(y - y.max()).sum()) + y.max()
             lg[b, i] = np.float32((R - np.log(rest)) * T[b])
+            if shape == "low" and b % 2:
+                p[b] = rng.uniform(0.98, 0.9999)        # a cut at the end of the row, or none
             if shape == "dominated" and p[b] < 1.0:     # (at 1 such a draw may miss the sum: not planned)
                 u[b] = rng.choice([u[b], np.float32(1.0 - 1e-4)])
     return lg, T, p, rep, rec, u
