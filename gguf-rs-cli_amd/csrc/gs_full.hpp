@@ -101,6 +101,19 @@ __device__ __forceinline__ int f_bin(float dp)
     const int b = (int)((kFDUp - dp) * kFInvW);
     return min(max(b, 0), kFBins - 1);
 }
+// x / T from iT = 1 / T rounded to double: three instructions for an element
+// where the division of floats takes a dozen, and pass 1, 2 and 3 scale every
+// element.  The product is within 2^-52 of x / T, and a quotient of two floats
+// that is a normal float is no midpoint of two floats and lies 2^-49 or
+// more from the next one, so rounding the product to float gives x / T
+// itself (infinities, zeros, NaN and overflow too).  A quotient below 2^-126
+// may be one of its steps (2^-149) off where it is a midpoint; no summand
+// sees that: y - m rounds to -m, or is so small that its exp is 1.
+// Where the passes are bound by issue: 8 rows at V 50257 129.8 -> 124.9 us
+// (passes 2 and 3 18.7 + 13.2 -> 17.0 + 10.7 us), 300 rows at V 100000
+// 317 -> 300 us, 512 mixed rows at V 256000 351 -> 329 us.  256 rows at
+// V 152064 stay at 230..233 us: their passes wait for the caches (4 TB/s).
+__device__ __forceinline__ float f_scaled(float x, double iT) { return (float)((double)x * iT); }
 __device__ __forceinline__ uint64_t f_entry(float y, uint32_t i) { return ((uint64_t)f2key(y) << 32) | (uint64_t)(~i); }
 __device__ __forceinline__ float f_entry_y(uint64_t en) { return key2f((uint32_t)(en >> 32)); }
 __device__ __forceinline__ uint32_t f_entry_id(uint64_t en) { return ~(uint32_t)en; }
@@ -1101,7 +1114,8 @@ __device__ bool full_v2_row(RowSmem &sm, const float *row, int V, float T, float
     const float4 *r4 = reinterpret_cast<const float4 *>(row + h0);
     const int n4 = (V - h0) >> 2;
     if (V < h0 || n4 == 0) F_FAIL();
-    auto ydiv = [&](float x) { return t_one ? x : x / T; };
+    const double iT = 1.0 / (double)T;
+    auto ydiv = [&](float x) { return t_one ? x : f_scaled(x, iT); };
     auto pen_y = [&](int s) { return ydiv(__uint_as_float(sm.hval[s])); };
 
     for (int b = t; b < kFBins; b += kThreads) { f.cnt[b] = 0u; f.v1[b] = 0u; }
@@ -1155,7 +1169,7 @@ __device__ bool full_v2_row(RowSmem &sm, const float *row, int V, float T, float
         }
         return true;
     };
-    if (!(t_one ? pass1([](float x) { return x; }) : pass1([&](float x) { return x / T; }))) F_FAIL();
+    if (!(t_one ? pass1([](float x) { return x; }) : pass1([&](float x) { return f_scaled(x, iT); }))) F_FAIL();
     for (int i = h0 + (n4 << 2) + t; i < V; i += kThreads) visit1(i, ydiv(ldg(row + i)));
     if (t < h0) visit1(t, ydiv(ldg(row + t)));
     if (has_pen) {
@@ -1351,7 +1365,7 @@ __device__ bool full_v2_row(RowSmem &sm, const float *row, int V, float T, float
     // entries written here instead of evicting them half-written; measured,
     // the fetches of pass 3 do not grow)
     if (t_one) row_for_each_any<true>(row, V, visit2);
-    else row_for_each_any<true>(row, V, [&](int i, float x) { visit2(i, x / T); });
+    else row_for_each_any<true>(row, V, [&](int i, float x) { visit2(i, f_scaled(x, iT)); });
     __syncthreads();
     if (has_pen) {
         // the raw values of penalized ids leave: listed entries are zeroed,
@@ -1634,7 +1648,7 @@ __device__ bool full_v2_row(RowSmem &sm, const float *row, int V, float T, float
     // (the row's last pass: non-temporal loads, so the row does not push the
     // partly written list lines out of L2)
     if (t_one) row_for_each_any<true>(row, V, [&](int i, float y) { visit3(i, y, 0u); });
-    else row_for_each_any<true>(row, V, [&](int i, float x) { visit3(i, x / T, 0u); });
+    else row_for_each_any<true>(row, V, [&](int i, float x) { visit3(i, f_scaled(x, iT), 0u); });
     __syncthreads();
     if (has_pen) {
         for (int s = t; s < kHashSlots; s += kThreads) {

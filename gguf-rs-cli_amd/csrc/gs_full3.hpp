@@ -881,7 +881,8 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
     const float4 *r4 = reinterpret_cast<const float4 *>(row + h0);
     const int n4 = (V - h0) >> 2;
     if (V < h0 || n4 == 0) F3_FAIL();
-    auto ydiv = [&](float x) { return t_one ? x : x / T; };
+    const double iT = 1.0 / (double)T;
+    auto ydiv = [&](float x) { return t_one ? x : f_scaled(x, iT); };
     auto pen_y = [&](int s) { return ydiv(__uint_as_float(sm.hval[s])); };
 
     for (int b = t; b < kF3Tab; b += kThreads) f.w[b] = 0u;
@@ -975,7 +976,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
 #endif
         return true;
     };
-    if (!(t_one ? pass1([](float x) { return x; }) : pass1([&](float x) { return x / T; }))) F3_FAIL();
+    if (!(t_one ? pass1([](float x) { return x; }) : pass1([&](float x) { return f_scaled(x, iT); }))) F3_FAIL();
     for (int i = h0 + (n4 << 2) + t; i < V; i += kThreads) visit1(i, ydiv(ldg(row + i)));
     if (t < h0) visit1(t, ydiv(ldg(row + t)));
     if (has_pen) {
@@ -1279,7 +1280,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
         auto act = [](uint32_t w) { return w != 0u; };
         uint2 *ring = reinterpret_cast<uint2 *>(f.u.w23) + 256 * wave_id();
         if (t_one) f3_qpass<256, false>(row, V, [](float x) { return x; }, word, act, one, ring, &f.qctr[0]);
-        else f3_qpass<256, false>(row, V, [&](float x) { return x / T; }, word, act, one, ring, &f.qctr[0]);
+        else f3_qpass<256, false>(row, V, [&](float x) { return f_scaled(x, iT); }, word, act, one, ring, &f.qctr[0]);
         __syncthreads();
         if (has_pen) {
             // the raw values of penalized ids leave (the pass marked their
@@ -1640,7 +1641,7 @@ __device__ bool full_v3_row(RowSmem &sm, const float *row, int V, float T, float
         auto act = [](uint2 w) { return (w.x | w.y) != 0u; };
         uint2 *ring = reinterpret_cast<uint2 *>(f.pre) + 128 * wave_id();
         if (t_one) f3_qpass<128, true>(row, V, [](float x) { return x; }, word, act, one, ring, &f.qctr[1]);
-        else f3_qpass<128, true>(row, V, [&](float x) { return x / T; }, word, act, one, ring, &f.qctr[1]);
+        else f3_qpass<128, true>(row, V, [&](float x) { return f_scaled(x, iT); }, word, act, one, ring, &f.qctr[1]);
         __syncthreads();
         F3_TS(10);
         if (has_pen) {
