@@ -6,23 +6,31 @@
 // Two kernels, for up to 4 vectors and for more, on the matrix cores, for
 // every type and row length.  The stored integers of a weight are exact in
 // f16 (at most 8 bits; Q3_K's scaled by its 6-bit sub-block scale: at most
-// 9), and x is split into two f16 parts, x s = hi + lo with s a power of two,
-// whose products the MFMA adds in f32.  What is left for the vector units is
-// the unpacking of the integers (about 1.3 instructions per weight for the
-// 4-bit types) and a multiply-add per sub-block, row and vector.
+// 9), and x is split into three f16 parts that hold its 24 bits, whose
+// products the MFMA adds in f32.  What is left for the vector units is the
+// unpacking of the integers (about 1.3 instructions per weight for the 4-bit
+// types) and, per sub-block, row and vector, an addition and a multiply-add.
 //
 // Why: the weights have to be read once per call, and that read is the bound
-// up to about 16 vectors.  Byte-to-float conversions and FMAs took 3.2-3.4
+// for a few vectors.  Byte-to-float conversions and FMAs took 3.2-3.4
 // instructions per weight, as long as the read itself, for one vector, and a
 // pass over the weights for each further one.  Measured (MI355X, us per call;
-// before: one pass per vector):
-//   Q4_K 152064 x 3584:  1 vector 61-68 -> 50 (6.1 TB/s), 16: 980 -> 77,
-//                        32: 1960 -> 115
-//   Q6_K 152064 x 3584:  1 vector 72.4 -> 72.6 (6.2 TB/s), 32: 2340 -> 160
-//   Q5_K 32000 x 8192:   1 vector 121 -> 38
-//   Q8_0 32000 x 4096:   4 vectors 100 -> 23
-// The error against 64-bit sums is 1.0e-7 to 2.0e-7 (2-norm, relative) where
-// it was 1.3e-7 to 2.1e-7.
+// before: one pass of the vector units per vector):
+//   Q4_K 152064 x 3584:  1 vector 62 -> 57 (5.5 TB/s), 16: 980 -> 93,
+//                        32: 1970 -> 145
+//   Q6_K 152064 x 3584:  1 vector 72 -> 77 (5.8 TB/s), 16: 1160 -> 144,
+//                        32: 2330 -> 231
+//   Q5_K 32000 x 8192:   1 vector 120 -> 40
+//   Q8_0 32000 x 4096:   4 vectors 95 -> 25
+// With x in two parts (23 bits at best) instead of three and their products
+// in one sum: 51, 78 and 115 us for Q4_K, 72, 108 and 160 for Q6_K.
+//
+// Error against 64-bit sums (2-norm, relative; x normal, channels of unequal
+// size; 1024, 3584 and 8192 columns, 1 to 32 vectors), before -> now:
+//   Q4_0 2.2-2.5e-7 -> 0.7-1.0e-7     Q4_K 1.3-1.5e-7 -> 0.9-1.2e-7
+//   Q4_1 1.8-2.1e-7 -> 1.3-1.7e-7     Q5_K 1.2-1.5e-7 -> 0.8-1.2e-7
+//   Q8_0 2.0-2.2e-7 -> 0.8-1.1e-7     Q6_K 2.0-2.2e-7 -> 0.9-1.2e-7
+//   Q3_K 1.8-2.0e-7 -> 0.8-1.1e-7
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>
@@ -105,11 +113,9 @@ __device__ __forceinline__ h2_t u4(uint32_t w, float off) { return n4(and_or(w, 
 // ------------------------------------------------------- operand layouts ---
 // v_mfma_f32_16x16x32_f16, lane L = 16 g + n: operand A holds row n, k = 8 g
 // .. 8 g + 7 (x); operand B column n, the same k (weight row n of the tile);
-// D column n, rows 4 g .. 4 g + 3.  (16x16x16: k = 4 g .. 4 g + 3.)  With the
-// weights as B, everything of a weight row (bits, scales, sums) sits in the
-// lanes with that n.
+// D column n, rows 4 g .. 4 g + 3.  With the weights as B, everything of a
+// weight row (bits, scales, sums) sits in the lanes with that n.
 __device__ __forceinline__ f4_t mfma(h8_t a, h8_t b, f4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f4_t mfma(h4_t a, h4_t b, f4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
 constexpr f4_t kZero = {0.0f, 0.0f, 0.0f, 0.0f};
 
 // ------------------------------------------------------------- formats -----
@@ -122,13 +128,11 @@ constexpr f4_t kZero = {0.0f, 0.0f, 0.0f, 0.0f};
 //          or 32 ks + 8 g .. + 7;
 //   kSwap  within four columns the unpacked order is 0, 2, 1, 3 (bytes 0 and
 //          2 of a word, then 1 and 3);
-//   kHalf  a scale for each 16 columns, and an operand for each (their first
-//          four columns of a lane, and the other four);
-//   kChain the sub-block scales are in the operands;
+//   kHalf  a scale for each 16 columns (a lane's first four of a step, and the
+//          other four), so a sum for each;
 //   kRecScale a factor of the whole record, rec();
 //   kMin   a term min_scale() * (min_frag() . the sums of x over 32 columns);
-//   Item, load(); frag(): the operand of a step (and half of it); sub(): its
-//          scale;
+//   Item, load(); frag(): the operand of a step; sub(): its scale (its half's);
 //   put(): a lane's part of a record from the 256 (or 8 x 32) GGUF blocks of
 //          its row.
 
@@ -157,7 +161,7 @@ __device__ __forceinline__ h2_t two(uint32_t w, int i, float off)
 // byte l of a block's 16 holds weight l (low nibble) and l + 16 (high).
 template <bool Q41> struct Q4Fmt {
     static constexpr int kRec = 2048 + 256 + (Q41 ? 256 : 0), kBlock = Q41 ? 20 : 18, kCols = 32;
-    static constexpr bool kSplit = true, kSwap = true, kHalf = false, kChain = false, kRecScale = false, kMin = Q41;
+    static constexpr bool kSplit = true, kSwap = true, kHalf = false, kRecScale = false, kMin = Q41;
     struct Item { u4_t q[2], d, m; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -192,7 +196,7 @@ template <bool Q41> struct Q4Fmt {
 // Q8_0: w = q d, int8 q, stored as q + 128.
 struct Q8Fmt {
     static constexpr int kRec = 4096 + 256, kBlock = 34, kCols = 32;
-    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kChain = false, kRecScale = false, kMin = false;
+    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kRecScale = false, kMin = false;
     struct Item { u4_t q[4], d; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -240,7 +244,7 @@ __device__ inline uint32_t k4_min(const Src &s, int o, int j)
 // the nibbles.
 template <bool Q5> struct KFmt {
     static constexpr int kRec = 2048 + (Q5 ? 512 : 0) + 256 + 64, kBlock = Q5 ? 176 : 144, kCols = 256;
-    static constexpr bool kSplit = false, kSwap = true, kHalf = false, kChain = false, kRecScale = true, kMin = true;
+    static constexpr bool kSplit = false, kSwap = true, kHalf = false, kRecScale = true, kMin = true;
     struct Item { u4_t q[2]; u2_t h, sc, mn; uint32_t dd; };
     static constexpr int kH = 2048, kS = 2048 + (Q5 ? 512 : 0), kM = kS + 128, kD = kS + 256;
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
@@ -312,7 +316,7 @@ template <bool Q5> struct KFmt {
 // are summed apart and scaled in f32.
 struct Q6Fmt {
     static constexpr int kRec = 2048 + 1024 + 256 + 32, kBlock = 210, kCols = 256;
-    static constexpr bool kSplit = true, kSwap = true, kHalf = true, kChain = false, kRecScale = true, kMin = false;
+    static constexpr bool kSplit = true, kSwap = true, kHalf = true, kRecScale = true, kMin = false;
     struct Item { u4_t q[2], c, sc; uint32_t d; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -323,7 +327,7 @@ struct Q6Fmt {
         it.d = ld<uint16_t>(r, 3328 + 2 * (lane & 15));
     }
     // columns 16 i .. + 15 of step ks = 4 h + j
-    static __device__ __forceinline__ h4_t frag(const Item &it, int ks, int i)
+    static __device__ __forceinline__ h4_t half(const Item &it, int ks, int i)
     {
         const int h = ks >> 2, j = ks & 3;
         const uint32_t a = it.q[h][2 * (j & 1) + i], c = it.c[2 * h + i], e = j & 1 ? c << 2 : c << 4, f = j & 1 ? c >> 6 : c >> 4;
@@ -331,6 +335,11 @@ struct Q6Fmt {
                            n0(and_or(f, 0x00300030u, and_or(a >> 8, 0x000F000Fu, vreg(kMagic))), 32.0f))
                      : cat(n4(and_or(e, 0x03000300u, and_or(a, 0x00F000F0u, vreg(kMagic))), 32.0f),
                            n4(and_or(f, 0x03000300u, and_or(a >> 8, 0x00F000F0u, vreg(kMagic))), 32.0f));
+    }
+    static __device__ __forceinline__ h8_t frag(const Item &it, int ks)
+    {
+        const h4_t a = half(it, ks, 0), b = half(it, ks, 1);
+        return h8_t{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
     }
     // (an f16: two scales in two instructions, and the multiply-add takes it as it is)
     static __device__ __forceinline__ float sub(const Item &it, int ks, int i) { return (float)two(it.sc[ks >> 1], ks & 1, 128.0f)[i]; }
@@ -357,10 +366,10 @@ struct Q6Fmt {
 // nibble here (146 bytes per block on the device for the file's 110): a
 // lane's eight weights of a step are the nibbles 0, 4, 1, 5, 2, 6, 3, 7 of
 // its word.  |sc (u - 4)| <= 128 is exact in f16, so the scale goes into the
-// weights and a record is one chain of MFMAs.
+// weights.
 struct Q3Fmt {
     static constexpr int kRec = 2048 + 256 + 32, kBlock = 110, kCols = 256;
-    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kChain = true, kRecScale = true, kMin = false;
+    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kRecScale = true, kMin = false;
     struct Item { u4_t q[2]; u2_t sc; uint32_t d; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -408,47 +417,104 @@ struct Q3Fmt {
 };
 
 // ------------------------------------------------------- x in f16 parts ----
-// x s = hi + lo, s = 2^(13 - e) for the largest |x| in [2^e, 2^(e+1)) of the
-// columns that share s, and (kMin) the sums of x s over 32 columns, over 64,
-// in three parts.  The parts hold 22 bits of every x above 2^-24 of the
-// largest, and 2^-39 of the largest at worst.
+// x s = a + b + c, three f16 parts with their 11 bits each, s = 2^(15 - e)
+// for the largest |x| in [2^e, 2^(e+1)) of the record's 256 columns of the
+// vector.  Every x of at least 2^-16 of that largest is held exactly (24
+// bits: the parts are cut off, not rounded, and c has two bits left to hold);
+// a smaller one to half of f16's last step, 2^-40 of the largest.  (kMin) the
+// sums of x s over 32 columns, over 64, go into three parts too.
+//
+// A wave converts a record of a vector: lane L holds columns 4 L .. 4 L + 3,
+// those of step L / 8.
 __device__ __forceinline__ void x_scale(float mx, float &s, float &inv)
 {
-    // 2^(13 - e), at most 2^126, and its inverse (exact; e of a subnormal as
+    // 2^(15 - e), at most 2^126, and its inverse (exact; e of a subnormal as
     // -127, of an infinity as 128)
     const int e = (int)(__float_as_uint(mx) >> 23) - 127;
-    const int se = mx > 0.0f ? min(13 - e, 126) : 0;
+    const int se = mx > 0.0f ? min(15 - e, 126) : 0;
     s = __uint_as_float((uint32_t)(se + 127) << 23);
     inv = __uint_as_float((uint32_t)(127 - se) << 23);
 }
-// (For an infinite t the difference is a NaN, which the clamp drops: hi
-// alone decides the sum.)
-__device__ __forceinline__ void x_split(float t, _Float16 &hi, _Float16 &lo)
+__device__ __forceinline__ h2_t cut(float x, float y) { return __builtin_bit_cast(h2_t, __builtin_amdgcn_cvt_pkrtz(x, y)); }
+// (For an infinite t the difference is a NaN, which the clamp drops: a alone
+// decides the sum.)
+__device__ __forceinline__ float rest(float t, _Float16 a) { return __builtin_amdgcn_fmed3f(t - (float)a, -32.0f, 32.0f); }
+__device__ __forceinline__ void x_split2(float x, float y, h2_t (&q)[3])
 {
-    hi = (_Float16)t;
-    lo = (_Float16)__builtin_amdgcn_fmed3f(t - (float)hi, -4.0f, 4.0f);
+    q[0] = cut(x, y);
+    x = rest(x, q[0].x);
+    y = rest(y, q[0].y);
+    q[1] = cut(x, y);
+    q[2] = h2_t{(_Float16)(x - (float)q[1].x), (_Float16)(y - (float)q[1].y)};
 }
-__device__ __forceinline__ void x_split3(float t, _Float16 &a, _Float16 &b, _Float16 &c)
+// The value of a lane paired with this one (of 2, 4, 8 or 16 lanes that hold
+// equal halves).
+template <int C> __device__ __forceinline__ float pair(float x)
 {
-    a = (_Float16)t;
-    const float r = __builtin_amdgcn_fmed3f(t - (float)a, -4.0f, 4.0f);
-    b = (_Float16)r;
-    c = (_Float16)(r - (float)b);
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), C, 0xf, 0xf, true));
 }
-template <class F> constexpr int x_pos(int i)   // place of column i of four
+constexpr int kPair1 = 0xB1, kPair2 = 0x4E, kPair4 = 0x141, kPair8 = 0x140;    // quad_perm, row_half_mirror, row_mirror
+struct XRec {
+    h4_t q[3];          // the parts of the lane's columns, in operand order
+    _Float16 sum[3];    // (kMin) of the lane's step
+    float inv;          // 1 / s
+};
+template <class F> __device__ __forceinline__ XRec x_convert(f4_t x)
 {
-    return F::kSwap && (i == 1 || i == 2) ? 3 - i : i;
+    XRec r;
+    float mx = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+    mx = fmaxf(mx, pair<kPair1>(mx));
+    mx = fmaxf(mx, pair<kPair2>(mx));
+    mx = fmaxf(mx, pair<kPair4>(mx));
+    mx = fmaxf(mx, pair<kPair8>(mx));
+    const int b = __float_as_int(mx);
+    mx = fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(b, 0)), __int_as_float(__builtin_amdgcn_readlane(b, 16))),
+               fmaxf(__int_as_float(__builtin_amdgcn_readlane(b, 32)), __int_as_float(__builtin_amdgcn_readlane(b, 48))));
+    float s;
+    x_scale(mx, s, r.inv);
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] *= s;
+    h2_t u[3], v[3];
+    x_split2(x[0], x[F::kSwap ? 2 : 1], u);
+    x_split2(x[F::kSwap ? 1 : 2], x[3], v);
+#pragma unroll
+    for (int i = 0; i < 3; i++) r.q[i] = cat(u[i], v[i]);
+    if constexpr (F::kMin) {
+        float t = (x[0] + x[1]) + (x[2] + x[3]);
+        t += pair<kPair1>(t);
+        t += pair<kPair2>(t);
+        t += pair<kPair4>(t);
+        h2_t w[3];
+        x_split2(t * 0.015625f, 0.0f, w);
+#pragma unroll
+        for (int i = 0; i < 3; i++) r.sum[i] = w[i].x;
+    }
+    return r;
+}
+// Where a lane's columns of its step go: operand group g, half h of the eight.
+template <class F> __device__ __forceinline__ void x_place(int lane, int &g, int &h)
+{
+    const int i = lane & 7;     // columns 4 i .. 4 i + 3
+    g = F::kSplit ? i & 3 : i >> 1;
+    h = F::kSplit ? i >> 2 : i & 1;
 }
 
+// A step's sum: that of a's products with the weights (of a half's, kHalf)
+// from zero, that of c's from zero and of b's onto it, and the two added (an
+// MFMA that adds onto a sum cuts what falls below the largest term's last
+// bits, always downwards: a's products onto those of b and c, 1.6e-7 against
+// 64 bits for Q4_0 x 8192 where this has 1.1e-7).
+
 // ------------------------------------------------- up to 4 vectors (GEMV) ---
-// Rows 4 v, 4 v + 1 of A = hi, lo of vector v (the others zero): one MFMA per
-// step, and a lane's sum of vector g is D[0] + D[1].  Formats with a scale
-// for each 16 columns (kHalf) use all four rows: x of the first 16 columns
-// of the step in rows 4 v, 4 v + 1 (zeros for the others) and of the second
-// in 4 v + 2, 4 v + 3, so that D[2] + D[3] is the second half's sum.
+// Rows 4 v and 4 v + 1 of the first MFMA's A = parts a and c of vector v (the
+// others zero), row 4 v + 1 of the second one's = b: a lane's sums of vector
+// g are D[0] and D[1].  Formats with a scale for each 16 columns (kHalf) use
+// all four rows: x of the first 16 columns of the step (zeros for the others)
+// in 4 v and 4 v + 2, and of the second in 4 v + 1 and 4 v + 3.
 //
 // A block takes tpb tiles of 16 rows; its waves share the columns, a record
-// each, with their operands of x in registers for all tiles.  D tiles are in
+// each, with the operand of a and c in registers for all tiles and that of b
+// in LDS (both in registers take more than the 128 of 4 waves per SIMD).  D tiles are in
 // flight: a record's registers are loaded again, for the tile D further on,
 // as soon as it has been used.  The waves' sums meet in LDS every kBatch
 // tiles (two buffers: one barrier per batch); within a batch a wave's
@@ -456,11 +522,13 @@ template <class F> constexpr int x_pos(int i)   // place of column i of four
 // together (with equal priorities the youngest came late and ran the end of
 // each batch alone: Q4_K 152064 x 3584 59 us against 52, Q6_K 84 against 74).
 // Bound: the read of the weights (5.4-6.7 TB/s at 152064 x 3584).  Four tiles
-// in flight instead of two: 57 us against 52 (Q4_K).  Rows of more columns than the waves hold (MULTI) go in
-// chunks: a batch's tiles take one chunk after the other, the waves' sums
-// kept in LDS.
+// in flight instead of two: 57 us against 52 (Q4_K).  Rows of more columns
+// than the waves hold (MULTI) go in chunks: a batch's tiles take one chunk
+// after the other, the waves' sums kept in LDS.
 constexpr int kVecs = 4, kBatch = 8, kMaxWaves = 16, kInFlight = 2;
-constexpr int kXRow = 264, kXWave = 9 * kXRow + 112;    // f16s: a row of 256, padded; a wave's rows, zeros and sums
+// A wave's f16s of x in LDS: rows of 256, padded: two for each vector, one of
+// zeros for the unused rows of A, then [v][part][8] of the sums.
+constexpr int kXRow = 264, kXZeros = 2 * kVecs * kXRow, kXWave = (2 * kVecs + 1) * kXRow + 112;
 // floats of a tile's sums (16 more: the rows of four tiles in different banks)
 __host__ __device__ constexpr int lds_tile(int nw) { return nw * 64 + 16; }
 constexpr size_t gemv_lds(int nw)
@@ -469,95 +537,82 @@ constexpr size_t gemv_lds(int nw)
 }
 
 struct XOps {
-    h8_t f[8];
+    h8_t ac[8];
+    const _Float16 *b;  // in LDS, + 32 ks
     h8_t sx;
     float inv;          // 1 / s of vector g
 };
-
-// The operands of a record's columns [c0, c0 + 256): a lane converts columns
-// 4 L .. + 3 of each vector, and the parts meet in LDS.
+__device__ __forceinline__ void lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The operands of a record's columns [c0, c0 + 256) from the lane's columns
+// 4 L .. + 3 of each vector.  The parts pass through a vector's two rows of
+// LDS: a and c, then b stays in the second one; kHalf: the halves of a, of c
+// and of b, which stay, each with the other half's columns zero.
 template <class F>
 __device__ __forceinline__ void x_ops(XOps &o, const f4_t (&raw)[kVecs], _Float16 *lds, int nv, int cols, int c0)
 {
-    // row 2 v + part of the wave's LDS: the part's 256 f16s in operand order
-    // (step, g, 8); row 8: zeros, for the unused rows of A; then [v][part][8]
-    // of the sums
-    const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
-    _Float16 *sxs = lds + 9 * kXRow;
-    const int k = lane >> 3, c = (lane & 7) * 4;        // the lane's step, columns c .. c + 3 of it
-    const int at = 32 * k + (F::kSplit ? (c & 15) * 2 + (c >> 4) * 4 : c);
-    *reinterpret_cast<h4_t *>(lds + 8 * kXRow + 4 * lane) = h4_t{0, 0, 0, 0};
+    const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15, k = lane >> 3, q = m & 3;
+    const bool on = (m >> 2) < nv;
+    _Float16 *sxs = lds + kXZeros + kXRow;
+    int pg, ph;
+    x_place<F>(lane, pg, ph);
+    auto put = [&](int v, int row, h4_t x) {
+        *reinterpret_cast<h4_t *>(lds + (2 * v + row) * kXRow + 32 * k + 8 * pg + 4 * ph) = x;
+    };
+    auto from = [&](bool is, int row) { return lds + (on && is ? (2 * (m >> 2) + row) * kXRow : kXZeros) + 8 * g; };
+    const h4_t z = {0, 0, 0, 0};
+    *reinterpret_cast<h4_t *>(lds + kXZeros + 4 * lane) = z;
+    XRec r[kVecs];
     o.inv = 1.0f;
 #pragma unroll
     for (int v = 0; v < kVecs; v++)
         if (v < nv) {
-            const f4_t a = c0 + 4 * lane < cols ? raw[v] : kZero;
-            float mx = fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3])));
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-            float s, inv;
-            x_scale(mx, s, inv);
-            o.inv = g == v ? inv : o.inv;
-            h4_t hi, lo;
-            float sum = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float t = a[i] * s;
-                _Float16 h, l;
-                x_split(t, h, l);
-                hi[x_pos<F>(i)] = h;
-                lo[x_pos<F>(i)] = l;
-                sum += t;
-            }
-            *reinterpret_cast<h4_t *>(lds + 2 * v * kXRow + at) = hi;
-            *reinterpret_cast<h4_t *>(lds + (2 * v + 1) * kXRow + at) = lo;
-            if constexpr (F::kMin) {
-                sum += __shfl_xor(sum, 1, 64);
-                sum += __shfl_xor(sum, 2, 64);
-                sum += __shfl_xor(sum, 4, 64);
-                _Float16 p0, p1, p2;
-                x_split3(sum * 0.015625f, p0, p1, p2);
-                if ((lane & 7) < 3) sxs[24 * v + 8 * (lane & 7) + k] = (lane & 7) == 0 ? p0 : (lane & 7) == 1 ? p1 : p2;
-            }
+            r[v] = x_convert<F>(c0 + 4 * lane < cols ? raw[v] : kZero);
+            o.inv = g == v ? r[v].inv : o.inv;
+            if constexpr (F::kMin)
+                if ((lane & 7) < 3) sxs[24 * v + 8 * (lane & 7) + k] = (lane & 7) == 0 ? r[v].sum[0] : (lane & 7) == 1 ? r[v].sum[1] : r[v].sum[2];
+            put(v, F::kHalf ? ph : 0, r[v].q[0]);
+            put(v, F::kHalf ? 1 - ph : 1, F::kHalf ? z : r[v].q[2]);
         }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const bool on = (m >> 2) < nv && (F::kHalf || (m & 3) < 2);
-    const _Float16 *row = lds + (on ? 2 * (m >> 2) + (m & 1) : 8) * kXRow + 8 * g;
+    lds_fence();
+    const _Float16 *p = from(q < 2, q & 1);
 #pragma unroll
-    for (int ks = 0; ks < 8; ks++) {
-        h8_t h = *reinterpret_cast<const h8_t *>(row + 32 * ks);
-        if constexpr (F::kHalf) {
-            const h4_t z = {0, 0, 0, 0}, a = {h[0], h[1], h[2], h[3]}, b = {h[4], h[5], h[6], h[7]};
-            const h4_t c = m & 2 ? z : a, d = m & 2 ? b : z;
-            h = h8_t{c[0], c[1], c[2], c[3], d[0], d[1], d[2], d[3]};
-        }
-        o.f[ks] = h;
+    for (int ks = 0; ks < 8; ks++) o.ac[ks] = *reinterpret_cast<const h8_t *>(p + 32 * ks);
+    lds_fence();
+    if constexpr (F::kHalf) {
+#pragma unroll
+        for (int v = 0; v < kVecs; v++)
+            if (v < nv) put(v, ph, r[v].q[2]);
+        lds_fence();
+        p = from(q >= 2, q & 1);
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) o.ac[ks] = q >= 2 ? *reinterpret_cast<const h8_t *>(p + 32 * ks) : o.ac[ks];
+        lds_fence();
     }
+#pragma unroll
+    for (int v = 0; v < kVecs; v++)
+        if (v < nv) put(v, F::kHalf ? ph : 1, r[v].q[1]);
+    lds_fence();
+    o.b = F::kHalf ? from(q >= 2, q & 1) : from(q == 1, 1);
     if constexpr (F::kMin)      // (g = 3, other rows: zeros)
-        o.sx = *reinterpret_cast<const h8_t *>((m & 3) == 0 && (m >> 2) < nv && g < 3 ? sxs + 24 * (m >> 2) + 8 * g
-                                                                                         : lds + 8 * kXRow);
+        o.sx = *reinterpret_cast<const h8_t *>(on && q == 0 && g < 3 ? sxs + 24 * (m >> 2) + 8 * g : lds + kXZeros);
 }
 
 // A record's sum for the lane's row and vector, times s.
 template <class F> __device__ __forceinline__ float dot(const typename F::Item &it, const XOps &x)
 {
     float v = 0.0f;
-    f4_t D = kZero;
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
-        if constexpr (F::kHalf) {
-            const h4_t a = F::frag(it, ks, 0), b = F::frag(it, ks, 1);
-            D = mfma(x.f[ks], h8_t{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}, kZero);
-            v = fmaf(D[0] + D[1], F::sub(it, ks, 0), v);
-            v = fmaf(D[2] + D[3], F::sub(it, ks, 1), v);
-        } else {
-            D = mfma(x.f[ks], F::frag(it, ks), F::kChain ? D : kZero);
-            if constexpr (!F::kChain) v = fmaf(D[0] + D[1], F::sub(it, ks, 0), v);
-        }
+        const h8_t w = F::frag(it, ks);
+        const f4_t D = mfma(*reinterpret_cast<const h8_t *>(x.b + 32 * ks), w, mfma(x.ac[ks], w, kZero));
+        v = fmaf(D[0] + D[F::kHalf ? 2 : 1], F::sub(it, ks, 0), v);
+        if constexpr (F::kHalf) v = fmaf(D[1] + D[3], F::sub(it, ks, 1), v);
     }
-    if constexpr (F::kChain) v = D[0] + D[1];
     if constexpr (F::kRecScale) v *= F::rec(it);
     if constexpr (F::kMin) v = fmaf(mfma(x.sx, F::min_frag(it), kZero)[0], F::min_scale(it), v);
     return v;
@@ -575,14 +630,13 @@ qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
     _Float16 *xl = reinterpret_cast<_Float16 *>(red + 2 * kBatch * ts) + kXWave * w;
     XOps xo;
     typename F::Item it[kInFlight];
-    // past the block's tiles or the row's records: the last one, not used
-    auto load = [&](int d, int t, int p) {
+    auto load = [&](int d, int t, int p) {      // (past the block's tiles or the row's records: the last one, not used)
         F::load(it[d], opaque(W + ((size_t)min(t, t1 - 1) * np + min(p, np - 1)) * F::kRec), lane);
     };
     auto start = [&](int t, int p) {        // (x first: loads return in order)
         f4_t raw[kVecs];
 #pragma unroll
-        for (int v = 0; v < kVecs; v++)
+        for (int v = 0; v < kVecs; v++)     // (cols is a multiple of 32)
             raw[v] = *reinterpret_cast<const f4_t *>(x + (size_t)min(v, nv - 1) * cols + min(kPair * p + 4 * lane, cols - 4));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -641,106 +695,90 @@ qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
 }
 
 // ------------------------------------------- more vectors, up to 32 (GEMM) ---
-// VT tiles of 16 vectors: row m of A's tile vt is vector 16 vt + m, hi and lo
-// two MFMAs into one D, whose rows are the vectors.
+// VT tiles of 16 vectors: row m of A's tile vt is vector 16 vt + m, an MFMA
+// for each part of x, the rows of D (of a) and E (of b and c) the vectors.
 //
 // A block of 8 waves (one per CU, 2 waves per SIMD: 256 registers each) takes
 // up to 8 RT tiles of 16 rows at a time, RT to a wave, through all columns.
-// The x of a record is converted once per block into LDS (each wave a step of
-// all vectors; two buffers, one barrier per record) and read from there for
+// The x of a record is converted once per block into LDS (each wave 2 VT of
+// the vectors; two buffers, one barrier per record) and read from there for
 // two or three groups of the wave's tiles; a group's registers are loaded
 // again, for the next record, as soon as it has been used.  (x of 32 vectors
 // in registers for all columns would fill the CU's register file.)
-// Bound: the chain of a step in each wave (unpack, two MFMAs, additions) at
-// two waves per SIMD; VALU issue is 48% at 16 vectors.  Holding x in
-// registers as the kernel above does (up to 8 vectors in 128 registers, 16
-// with spills) took 74 us at 8 and 87 at 16 (Q4_K 152064 x 3584) where this
-// takes 74 and 77, and 158 for 32 in two passes where this takes 115.
 constexpr int kGemmWaves = 8;
-template <class F, int VT> constexpr int kXBuf = VT * (2 * 8 * 512 + (F::kMin ? 512 : 0));     // f16s of a record's x
+// f16s of a step's part in LDS: lane 16 g + m reads the eight at m, m ^ 8 in
+// the odd groups (so, and with the steps shifted by eight, the lanes that
+// write a vector's columns, four each, use all banks)
+constexpr int kXStep = 520;
+template <class F, int VT> constexpr int kXBuf = VT * (3 * 8 * kXStep + (F::kMin ? 512 : 0));     // of a record's x
+__device__ __forceinline__ int x_lane(int lane) { return 8 * (lane ^ (lane >> 1 & 8)); }
 
 template <class F, int VT, int N>
-__device__ __forceinline__ void group(const typename F::Item *it, const _Float16 *xb, float (*acc)[VT][4])
+__device__ __forceinline__ void group(const typename F::Item *it, const _Float16 *xb, const float *inv, float (*acc)[VT][4])
 {
     const int lane = threadIdx.x & 63;
-    xb += 8 * lane;
+    const _Float16 *xr = xb + x_lane(lane);
     float sum[N][VT][4] = {};   // of the record: shorter chains of additions
-    h8_t nh[VT], no[VT];        // the next step's x, read a step ahead
-    auto read = [&](int ks) {
+    h8_t nx[3];                 // the next vector tile's x, read ahead
+    auto read = [&](int ks, int v) {
 #pragma unroll
-        for (int v = 0; v < VT; v++) {
-            nh[v] = *reinterpret_cast<const h8_t *>(xb + (16 * v + ks) * 512);
-            no[v] = *reinterpret_cast<const h8_t *>(xb + (16 * v + 8 + ks) * 512);
-        }
+        for (int q = 0; q < 3; q++) nx[q] = *reinterpret_cast<const h8_t *>(xr + ((3 * v + q) * 8 + ks) * kXStep);
     };
-    read(0);
+    read(0, 0);
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
-        h8_t xh[VT], xo[VT];
+        h8_t f[N];
+        float s[N][2];
 #pragma unroll
-        for (int v = 0; v < VT; v++) { xh[v] = nh[v]; xo[v] = no[v]; }
-        if (ks < 7) read(ks + 1);
+        for (int r = 0; r < N; r++) {
+            f[r] = F::frag(it[r], ks);
 #pragma unroll
-        for (int r = 0; r < N; r++)
+            for (int i = 0; i < (F::kHalf ? 2 : 1); i++) s[r][i] = F::sub(it[r], ks, i);
+        }
 #pragma unroll
-            for (int i = 0; i < (F::kHalf ? 2 : 1); i++) {
-                const float s = F::sub(it[r], ks, i);
-#pragma unroll
-                for (int v = 0; v < VT; v++) {
-                    f4_t D;
-                    if constexpr (F::kHalf) {
-                        const h4_t b = F::frag(it[r], ks, i);
-                        D = mfma(h4_t{xh[v][4 * i], xh[v][4 * i + 1], xh[v][4 * i + 2], xh[v][4 * i + 3]}, b, kZero);
-                        D = mfma(h4_t{xo[v][4 * i], xo[v][4 * i + 1], xo[v][4 * i + 2], xo[v][4 * i + 3]}, b, D);
-                    } else {
-                        const h8_t b = F::frag(it[r], ks);
-                        D = mfma(xh[v], b, kZero);
-                        D = mfma(xo[v], b, D);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; j++) sum[r][v][j] = fmaf(D[j], s, sum[r][v][j]);
-                }
-            }
-        // a step's sums are done here (else the steps of a record are mixed
-        // until the registers spill)
-        if (VT == 2 || F::kHalf) {
+        for (int v = 0; v < VT; v++) {
+            const h8_t xa = nx[0], xb = nx[1], xc = nx[2];
+            if (v + 1 < VT) read(ks, v + 1);
+            else if (ks < 7) read(ks + 1, 0);
 #pragma unroll
             for (int r = 0; r < N; r++)
 #pragma unroll
-                for (int v = 0; v < VT; v++)
+                for (int i = 0; i < (F::kHalf ? 2 : 1); i++) {
+                    const h8_t w = !F::kHalf ? f[r] : i == 0 ? h8_t{f[r][0], f[r][1], f[r][2], f[r][3], 0, 0, 0, 0}
+                                                             : h8_t{0, 0, 0, 0, f[r][4], f[r][5], f[r][6], f[r][7]};
+                    const f4_t E = mfma(xb, w, mfma(xc, w, kZero)), D = mfma(xa, w, kZero);
 #pragma unroll
-                    for (int j = 0; j < 4; j++) asm volatile("" : "+v"(sum[r][v][j]));
+                    for (int j = 0; j < 4; j++) sum[r][v][j] = fmaf(D[j] + E[j], s[r][i], sum[r][v][j]);
+                }
+            // these sums are done here (else the steps of a record are mixed
+            // until the registers spill)
+#pragma unroll
+            for (int r = 0; r < N; r++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) asm volatile("" : "+v"(sum[r][v][j]));
             __builtin_amdgcn_sched_barrier(0);
         }
     }
     // The minimums join the record's own sum first: the two nearly cancel
     // where the weights are centred, and the running sum then takes the small
-    // difference (Q4_K 128256 x 4096, 16 vectors: 1.4e-7 -> 1.2e-7 against 64
-    // bits, 76.1 -> 74.4 us; 152064 x 3584, 32: 136.7 -> 129.2 us a decode step).
+    // difference.
 #pragma unroll
-    for (int r = 0; r < N; r++) {
-        const float s = F::rec(it[r]);
-        if (F::kRecScale && F::kMin) {
+    for (int v = 0; v < VT; v++) {
+        const f4_t iv = *reinterpret_cast<const f4_t *>(inv + 16 * v + 4 * (lane >> 4));
+        h8_t sx;
+        if constexpr (F::kMin) sx = *reinterpret_cast<const h8_t *>(xb + VT * 3 * 8 * kXStep + 512 * v + 8 * lane);
 #pragma unroll
-            for (int v = 0; v < VT; v++)
+        for (int r = 0; r < N; r++) {
+            f4_t D;
+            if constexpr (F::kMin) D = mfma(sx, F::min_frag(it[r]), kZero);
 #pragma unroll
-                for (int j = 0; j < 4; j++) sum[r][v][j] *= s;
-        }
-        if constexpr (F::kMin) {
-            const float ms = F::min_scale(it[r]);
-#pragma unroll
-            for (int v = 0; v < VT; v++) {
-                const h8_t sx = *reinterpret_cast<const h8_t *>(xb + (16 * VT + v) * 512);
-                const f4_t D = mfma(sx, F::min_frag(it[r]), kZero);
-#pragma unroll
-                for (int j = 0; j < 4; j++) sum[r][v][j] = fmaf(D[j], ms, sum[r][v][j]);
+            for (int j = 0; j < 4; j++) {
+                float t = sum[r][v][j];
+                if constexpr (F::kRecScale) t *= F::rec(it[r]);
+                if constexpr (F::kMin) t = fmaf(D[j], F::min_scale(it[r]), t);
+                acc[r][v][j] += t * iv[j];
             }
         }
-#pragma unroll
-        for (int v = 0; v < VT; v++)
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                acc[r][v][j] = F::kRecScale && !F::kMin ? fmaf(sum[r][v][j], s, acc[r][v][j]) : acc[r][v][j] + sum[r][v][j];
     }
     // The additions are done here: put off past the branches that follow they
     // keep the products of all steps in registers.
@@ -759,7 +797,7 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
     // RT > 1: the wave's tiles in groups of N; RT = 1: two records of its tile
     constexpr int N = RT <= 3 ? (RT + 1) / 2 : VT == 2 ? 2 : (RT + 1) / 2, NI = RT > 1 ? RT : 2;
     __shared__ __align__(16) _Float16 xs[2][kXBuf<F, VT>];
-    __shared__ float sc[VT * 16], si[VT * 16];
+    __shared__ __align__(16) float si[2][VT * 16];      // 1 / s of the vectors
     const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int v0 = blockIdx.y * per, nv = min(per, B - v0);
@@ -769,45 +807,29 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
     out += (size_t)v0 * rows;
 
     typename F::Item it[NI];
-    f4_t raw[2 * VT];
-    const float *xv[VT];
+    f4_t raw[2 * VT];           // columns 4 lane .. + 3 of vectors w, w + 8, ..
+    auto xload = [&](int p) {   // (cols is a multiple of 32)
+        const int c = min(kPair * p + 4 * lane, cols - 4);
 #pragma unroll
-    for (int v = 0; v < VT; v++) xv[v] = x + (size_t)min(16 * v + m, nv - 1) * cols + (F::kSplit ? 4 * g : 8 * g);
-    auto xload = [&](int p) {       // step w of record p
-        const int c = min(kPair * p + 32 * w, cols - 32);
-#pragma unroll
-        for (int v = 0; v < VT; v++) {
-            raw[2 * v] = *reinterpret_cast<const f4_t *>(xv[v] + c);
-            raw[2 * v + 1] = *reinterpret_cast<const f4_t *>(xv[v] + c + (F::kSplit ? 16 : 4));
-        }
+        for (int i = 0; i < 2 * VT; i++) raw[i] = *reinterpret_cast<const f4_t *>(x + (size_t)min(w + 8 * i, nv - 1) * cols + c);
     };
-    float s[VT];
+    int pg, ph;
+    x_place<F>(lane, pg, ph);
+    const int at = (lane >> 3) * kXStep + 4 * ph;
     auto xput = [&](int p) {
-        _Float16 *b = xs[p & 1] + 8 * lane;
+        _Float16 *b = xs[p & 1];
 #pragma unroll
-        for (int v = 0; v < VT; v++) {
-            const bool in = 16 * v + m < nv && kPair * p + 32 * w < cols;
-            h8_t hi, lo;
-            float sum = 0.0f;
+        for (int i = 0; i < 2 * VT; i++) {
+            const int v = w + 8 * i, vt = i >> 1, vm = v & 15;
+            const XRec r = x_convert<F>(v < nv && kPair * p + 4 * lane < cols ? raw[i] : kZero);
 #pragma unroll
-            for (int h = 0; h < 2; h++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float t = in ? raw[2 * v + h][i] * s[v] : 0.0f;
-                    _Float16 a, c;
-                    x_split(t, a, c);
-                    hi[4 * h + x_pos<F>(i)] = a;
-                    lo[4 * h + x_pos<F>(i)] = c;
-                    sum += t;
-                }
-            *reinterpret_cast<h8_t *>(b + (16 * v + w) * 512) = hi;
-            *reinterpret_cast<h8_t *>(b + (16 * v + 8 + w) * 512) = lo;
-            if constexpr (F::kMin) {        // lanes 16 g + m hold part g of the sum over the step
-                sum += __shfl_xor(sum, 16, 64);
-                sum += __shfl_xor(sum, 32, 64);
-                _Float16 a0, a1, a2;
-                x_split3(sum * 0.015625f, a0, a1, a2);
-                b[(16 * VT + v) * 512 + w] = g == 0 ? a0 : g == 1 ? a1 : g == 2 ? a2 : (_Float16)0.0f;
+            for (int q = 0; q < 3; q++) *reinterpret_cast<h4_t *>(b + (3 * vt + q) * 8 * kXStep + at + x_lane(16 * pg + vm)) = r.q[q];
+            if (lane == 0) si[p & 1][v] = r.inv;
+            if constexpr (F::kMin) {        // lanes 16 g + m hold part g of the sums over the steps
+                const int q = lane & 7;
+                if (q < 4)
+                    b[VT * 3 * 8 * kXStep + 512 * vt + 8 * (16 * q + vm) + (lane >> 3)] =
+                        q == 0 ? r.sum[0] : q == 1 ? r.sum[1] : q == 2 ? r.sum[2] : (_Float16)0.0f;
             }
         }
     };
@@ -817,7 +839,6 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
 
-    bool first = true;
     const int rounds = (t1 - t0 + kGemmWaves * RT - 1) / (kGemmWaves * RT);
     for (int rd = 0; rd < rounds; rd++) {
         // the round's tiles, spread evenly over the waves
@@ -830,36 +851,16 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
         xload(0);
 #pragma unroll
         for (int i = 0; i < NI; i++) load(i, RT > 1 ? i : 0, RT > 1 ? 0 : i);
-        if (first) {        // the scale of each vector, from all its columns
-            for (int v = w; v < 16 * VT; v += kGemmWaves) {
-                float mx = 0.0f;
-                if (v < nv) {
-                    const float *p = x + (size_t)v * cols;
-                    for (int c = 4 * lane; c < cols; c += 256) {
-                        const f4_t a = *reinterpret_cast<const f4_t *>(p + c);
-                        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))));
-                    }
-                }
-#pragma unroll
-                for (int d = 1; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-                float a, b;
-                x_scale(mx, a, b);
-                if (lane == 0) { sc[v] = a; si[v] = b; }
-            }
-            sync();
-            first = false;
-#pragma unroll
-            for (int v = 0; v < VT; v++) s[v] = sc[16 * v + m];
-        }
         float acc[RT][VT][4] = {};
         xput(0);
         xload(1);
         sync();
         for (int p = 0; p < np; p += RT > 1 ? 1 : 2) {
             const _Float16 *xb = xs[p & 1];
+            const float *sb = si[p & 1];
             __builtin_amdgcn_s_setprio(3);
             __builtin_amdgcn_sched_barrier(0);
-            group<F, VT, N>(it, xb, acc);
+            group<F, VT, N>(it, xb, sb, acc);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < N; i++) load(i, i, p + (RT > 1 ? 1 : 2));
@@ -872,8 +873,8 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
                     if (r == N) __builtin_amdgcn_s_setprio(1);
                     else __builtin_amdgcn_s_setprio(0);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (M == 0 || r + N <= RT) group<F, VT, N>(it + r, xb, acc + r);
-                    else group<F, VT, M ? M : 1>(it + r, xb, acc + r);
+                    if (M == 0 || r + N <= RT) group<F, VT, N>(it + r, xb, sb, acc + r);
+                    else group<F, VT, M ? M : 1>(it + r, xb, sb, acc + r);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int i = r; i < r + N; i++)
@@ -883,7 +884,7 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
                 sync();
                 float t[1][VT][4] = {};         // (past the last record: not used)
                 __builtin_amdgcn_sched_barrier(0);
-                group<F, VT, 1>(it + 1, xs[1], t);
+                group<F, VT, 1>(it + 1, xs[1], si[1], t);
                 __builtin_amdgcn_sched_barrier(0);
                 load(1, 0, p + 3);
 #pragma unroll
@@ -900,12 +901,11 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int vec = 16 * v + 4 * g + j;
-                const float inv = si[vec];
 #pragma unroll
                 for (int r = 0; r < RT; r++) {
                     const uint32_t row = 16u * (tw + r) + m;
                     if (r < cnt && vec < nv && row < (uint32_t)rows)
-                        __builtin_nontemporal_store(acc[r][v][j] * inv, out + (size_t)vec * rows + row);
+                        __builtin_nontemporal_store(acc[r][v][j], out + (size_t)vec * rows + row);
                 }
             }
     }
@@ -1018,7 +1018,6 @@ int gemm(const gs_qmatrix *m, const float *x, float *out, int B, int per, int gr
     if (blocks < 1) blocks = 1;
     const int tpb = (m->tiles + blocks - 1) / blocks;
     blocks = (m->tiles + tpb - 1) / tpb;
-    // rounds of at most 5 tiles per wave, as even as they can be
     const int rounds = (tpb + 5 * gs::kGemmWaves - 1) / (5 * gs::kGemmWaves);
     const int rt = ((tpb + rounds - 1) / rounds + gs::kGemmWaves - 1) / gs::kGemmWaves;
     switch (rt) {

@@ -87,9 +87,10 @@ int gs_qmatrix_shape(const gs_qmatrix *m, uint32_t *qtype, size_t *rows, size_t 
  * d_out[b*rows + r] = sum_c W[r][c] * d_x[b*cols + c].  Device pointers;
  * asynchronous on `stream` (NULL = default stream).  B = 1 is the reference's
  * decode step; up to 32 vectors share one pass over the weights (the matrix
- * cores take them together; x is split into two f16 parts whose products are
- * added in f32, with an error no larger than that of f32 arithmetic), larger
- * B goes in groups of up to 32.  An infinity or NaN in a vector makes its own
+ * cores take them together), larger B goes in groups of up to 32.  The sums
+ * are f32; x is split into three f16 parts, which hold all 24 bits of every
+ * value of at least 2^-16 of the largest of its 256 columns (256 k .. 256 k +
+ * 255 of one vector), and a smaller one to 2^-40 of that largest.  An infinity or NaN in a vector makes its own
  * logits non-finite and no other vector's. */
 int gs_gemv(const gs_qmatrix *m, const float *d_x, size_t B, float *d_out, void *stream);
 

@@ -468,6 +468,72 @@ def test_gemv_vectors(gpu, torch, oracle, qt, rows, cols, B):
     _gpu_check(gpu, torch, oracle, qt, rows, cols, seed=rows + cols + B, B=B, x_kind="spiky")
 
 
+def _unit_blocks(qt, rows, cols, at):
+    """Blocks of a matrix whose row r is 1 at column at[r] and 0 elsewhere."""
+    import workloads
+    w, nb = workloads.QBLOCK[qt]
+    b = np.zeros((rows, cols // w, nb), np.uint8)
+    one = np.array([1.0], np.float16).view(np.uint8)
+    r, j, c = np.arange(rows), np.asarray(at) // w, np.asarray(at) % w
+    b[:, :, {Q3_K: 108, Q6_K: 208}.get(qt, 0):][:, :, :2] = one
+    if qt == Q8_0:
+        b[r, j, 2 + c] = 1
+    elif qt in (Q4_0, Q4_1):
+        o = 4 if qt == Q4_1 else 2
+        if qt == Q4_0:
+            b[:, :, o:] = 0x88                                   # q - 8
+        b[r, j, o + c % 16] += np.where(c < 16, 1, 16).astype(np.uint8)
+    elif qt in (Q4_K, Q5_K):
+        b[:, :, 4:8] = 1                                         # scales 1, minimums 0
+        b[:, :, 12:16] = 1
+        b[r, j, (48 if qt == Q5_K else 16) + 32 * (c // 64) + c % 32] = np.where(c % 64 < 32, 1, 16)
+    elif qt == Q6_K:
+        b[:, :, 128:192] = 0xAA                                  # u = 32
+        b[:, :, 192:208] = 1
+        b[r, j, 64 * (c // 128) + 32 * (c // 32 % 2) + c % 32] = np.where(c % 128 < 64, 1, 16)
+    else:
+        b[:, :, 0:32] = 0xFF                                     # u = 4
+        b[:, :, 96:104] = 0x11                                   # scales 33 - 32
+        b[:, :, 104:108] = 0xAA
+        b[r, j, 32 + 32 * (c // 128) + c % 32] = 1 << (2 * (c // 32 % 4))
+    return b.reshape(-1)
+
+
+@pytest.mark.parametrize("qt", ALL_TYPES)
+def test_unit_blocks(oracle, qt):
+    at = np.random.default_rng(qt).permutation(512)
+    w = oracle.dequant(qt, _unit_blocks(qt, 512, 512, at), 512 * 512).reshape(512, 512)
+    assert np.array_equal(w, np.eye(512, dtype=np.float32)[at])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", ALL_TYPES)
+@pytest.mark.parametrize("B", [1, 4, 5, 16, 17, 32])
+def test_gemv_x_is_whole(gpu, torch, qt, B):
+    """All 24 bits of x reach the result: with one weight of 1 per row the
+    logits are x itself, bit for bit, for every x of at least 2^-16 of the
+    largest of its record (256 columns).  A value 2^20 times the others, where
+    these weights are 0, costs the other records nothing, and its own at most
+    2^-40 of it."""
+    n = 768
+    rng = np.random.default_rng(100 * qt + B)
+    x = rng.standard_normal((B, n)).astype(np.float32)
+    x[np.abs(x) < 2.0 ** -10] += np.float32(0.37)
+    m = gpu.QMatrix(qt, _unit_blocks(qt, n, n, np.arange(n)), n, n)
+    d_o = torch.zeros((B, n), device="cuda")
+    print("gemv x", qt, B, flush=True)
+    m.gemv(torch.from_numpy(x).cuda(), d_o, B=B)
+    assert np.array_equal(_f32_bits(d_o.cpu().numpy()), _f32_bits(x))
+    x[:, 300] *= np.float32(1.37 * 2.0 ** 20) / np.abs(x).max()
+    m.gemv(torch.from_numpy(x).cuda(), d_o, B=B)
+    got = d_o.cpu().numpy()
+    m.close()
+    own = np.arange(n) // 256 == 1
+    assert np.array_equal(_f32_bits(got[:, ~own]), _f32_bits(x[:, ~own]))
+    big = np.abs(x[:, own]).max(1, keepdims=True).astype(np.float64)
+    assert (np.abs(got[:, own].astype(np.float64) - x[:, own]) <= 2.0 ** -40 * big).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("qt,cols", [(Q4_0, 32), (Q4_0, 288), (Q4_1, 96), (Q8_0, 480), (Q8_0, 2016)])
 @pytest.mark.parametrize("B", [1, 7, 20])
