@@ -499,11 +499,15 @@ template <class F> __device__ __forceinline__ void x_place(int lane, int &g, int
     h = F::kSplit ? i >> 2 : i & 1;
 }
 
-// A step's sum: that of a's products with the weights (of a half's, kHalf)
-// from zero, that of c's from zero and of b's onto it, and the two added (an
-// MFMA that adds onto a sum cuts what falls below the largest term's last
-// bits, always downwards: a's products onto those of b and c, 1.6e-7 against
-// 64 bits for Q4_0 x 8192 where this has 1.1e-7).
+// The order of every addition is the same in the two kernels below, so a
+// vector's result does not depend on the others of the call: the sum of a's
+// products with a step's weights (of a half's, kHalf) from zero, that of c's
+// from zero and of b's onto it, and the two added (an MFMA that adds onto a
+// sum cuts what falls below the largest term's last bits, always downwards:
+// a's products onto those of b and c, 1.6e-7 against 64 bits for Q4_0 x 8192
+// where this has 1.1e-7); the steps of a record; the record's factor and its
+// minimums; record after record, kChunk at a time, and the chunks.
+constexpr int kChunk = 16;
 
 // ------------------------------------------------- up to 4 vectors (GEMV) ---
 // Rows 4 v and 4 v + 1 of the first MFMA's A = parts a and c of vector v (the
@@ -524,8 +528,8 @@ template <class F> __device__ __forceinline__ void x_place(int lane, int &g, int
 // Bound: the read of the weights (5.4-6.7 TB/s at 152064 x 3584).  Four tiles
 // in flight instead of two: 57 us against 52 (Q4_K).  Rows of more columns
 // than the waves hold (MULTI) go in chunks: a batch's tiles take one chunk
-// after the other, the waves' sums kept in LDS.
-constexpr int kVecs = 4, kBatch = 8, kMaxWaves = 16, kInFlight = 2;
+// after the other, and the running sums stay with the waves that add them.
+constexpr int kVecs = 4, kBatch = 8, kMaxWaves = kChunk, kInFlight = 2;
 // A wave's f16s of x in LDS: rows of 256, padded: two for each vector, one of
 // zeros for the unused rows of A, then [v][part][8] of the sums.
 constexpr int kXRow = 264, kXZeros = 2 * kVecs * kXRow, kXWave = (2 * kVecs + 1) * kXRow + 112;
@@ -630,8 +634,8 @@ qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
     _Float16 *xl = reinterpret_cast<_Float16 *>(red + 2 * kBatch * ts) + kXWave * w;
     XOps xo;
     typename F::Item it[kInFlight];
-    auto load = [&](int d, int t, int p) {      // (past the block's tiles or the row's records: the last one, not used)
-        F::load(it[d], opaque(W + ((size_t)min(t, t1 - 1) * np + min(p, np - 1)) * F::kRec), lane);
+    auto load = [&](int d, int t, int p) {      // (past the block's tiles: the last one, not used)
+        F::load(it[d], opaque(W + ((size_t)min(t, t1 - 1) * np + p) * F::kRec), lane);
     };
     auto start = [&](int t, int p) {        // (x first: loads return in order)
         f4_t raw[kVecs];
@@ -647,49 +651,49 @@ qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
     };
     if (!MULTI) start(t0, w);
     int buf = 0;
-    for (int tb = t0; tb < t1; tb += kBatch, buf ^= 1) {
+    for (int tb = t0; tb < t1; tb += kBatch) {
         const int nb = min(kBatch, t1 - tb);
-        float *rb = red + buf * kBatch * ts;
-        for (int c = 0; c < (MULTI ? np : 1); c += nw) {
+        float sum = 0.0f;       // of the chunks (MULTI: a wave adds for at most one vector and four tiles)
+        for (int c = 0; c < (MULTI ? np : 1); c += nw, buf ^= 1) {
+            float *rb = red + buf * kBatch * ts;
             const int p = c + w;
-            if (MULTI) start(tb, p);
-            for (int k0 = 0; k0 < nb; k0 += kInFlight) {
-                switch (k0 * 4 / kBatch) {
-                case 0: __builtin_amdgcn_s_setprio(3); break;
-                case 1: __builtin_amdgcn_s_setprio(2); break;
-                case 2: __builtin_amdgcn_s_setprio(1); break;
-                default: __builtin_amdgcn_s_setprio(0); break;
-                }
-#pragma unroll
-                for (int d = 0; d < kInFlight; d++) {       // (a tile past nb: not used)
-                    const int k = k0 + d;
-                    float v = dot<F>(it[d], xo) * xo.inv;
-                    __builtin_amdgcn_sched_barrier(0);
-                    load(d, tb + k + kInFlight, p);
-                    float *q = rb + k * ts + w * 64 + lane;
-                    if (MULTI) {
-                        if (p >= np) v = 0.0f;
-                        if (c > 0) v += *q;
+            if (!MULTI || p < np) {
+                if (MULTI) start(tb, p);
+                for (int k0 = 0; k0 < nb; k0 += kInFlight) {
+                    switch (k0 * 4 / kBatch) {
+                    case 0: __builtin_amdgcn_s_setprio(3); break;
+                    case 1: __builtin_amdgcn_s_setprio(2); break;
+                    case 2: __builtin_amdgcn_s_setprio(1); break;
+                    default: __builtin_amdgcn_s_setprio(0); break;
                     }
-                    *q = v;
+#pragma unroll
+                    for (int d = 0; d < kInFlight; d++) {       // (a tile past nb: not used)
+                        const int k = k0 + d;
+                        const float v = dot<F>(it[d], xo) * xo.inv;
+                        __builtin_amdgcn_sched_barrier(0);
+                        load(d, tb + k + kInFlight, p);
+                        rb[k * ts + w * 64 + lane] = v;
+                    }
                 }
             }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        __builtin_amdgcn_s_setprio(3);
-        // a wave adds four tiles of a vector at a time: vector v, row n is in
-        // lane 16 v + n
-        for (int u = w; u < nv * (kBatch / 4); u += nw) {
-            const int v = u / (kBatch / 4), rr = (u % (kBatch / 4)) * 64 + lane;
-            const uint32_t r = 16u * tb + rr;
-            const float *q = rb + (rr >> 4) * ts + v * 16 + (lane & 15);
-            float s = 0.0f;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            __builtin_amdgcn_s_setprio(3);
+            // a wave adds four tiles of a vector at a time: vector v, row n is in
+            // lane 16 v + n
+            const int cnt = min(nw, np - c);
+            for (int u = w; u < nv * (kBatch / 4); u += nw) {
+                const int v = u / (kBatch / 4), rr = (u % (kBatch / 4)) * 64 + lane;
+                const uint32_t r = 16u * tb + rr;
+                const float *q = rb + (rr >> 4) * ts + v * 16 + (lane & 15);
+                float s = 0.0f;
 #pragma unroll
-            for (int i = 0; i < kMaxWaves; i++)
-                if (i < nw) s += q[i * 64];
-            if (rr < 16 * nb && r < (uint32_t)rows) out[(size_t)v * rows + r] = s;
+                for (int i = 0; i < kMaxWaves; i++)
+                    if (i < cnt) s += q[i * 64];
+                if (MULTI) sum = s = c > 0 ? sum + s : s;
+                if (c + nw >= np && rr < 16 * nb && r < (uint32_t)rows) out[(size_t)v * rows + r] = s;
+            }
         }
     }
 }
@@ -852,6 +856,29 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
 #pragma unroll
         for (int i = 0; i < NI; i++) load(i, RT > 1 ? i : 0, RT > 1 ? 0 : i);
         float acc[RT][VT][4] = {};
+        // The sums of a chunk that ends before record p: onto those of the
+        // chunks before it, which wait in out.
+        auto flush = [&](int p) {
+            // (opaque: else the addresses and conditions are kept in registers through the loop)
+            size_t ld = rows;
+            int lim = nv, most = cnt;
+            asm volatile("" : "+s"(ld), "+s"(lim), "+s"(most));
+#pragma unroll
+            for (int v = 0; v < VT; v++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int vec = 16 * v + 4 * g + j;
+#pragma unroll
+                    for (int r = 0; r < RT; r++) {
+                        const uint32_t row = 16u * (tw + r) + m;
+                        if (r < most && vec < lim && row < ld) {
+                            float *o = out + vec * ld + row;
+                            __builtin_nontemporal_store(p > kChunk ? *o + acc[r][v][j] : acc[r][v][j], o);
+                        }
+                        acc[r][v][j] = 0.0f;
+                    }
+                }
+        };
         xput(0);
         xload(1);
         sync();
@@ -882,32 +909,19 @@ qgemm_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
                 }
             } else {
                 sync();
-                float t[1][VT][4] = {};         // (past the last record: not used)
-                __builtin_amdgcn_sched_barrier(0);
-                group<F, VT, 1>(it + 1, xs[1], si[1], t);
-                __builtin_amdgcn_sched_barrier(0);
-                load(1, 0, p + 3);
-#pragma unroll
-                for (int v = 0; v < VT; v++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) acc[0][v][j] += p + 1 < np ? t[0][v][j] : 0.0f;
-                xput(p + 2);
-                xload(p + 3);
-            }
-            sync();
-        }
-#pragma unroll
-        for (int v = 0; v < VT; v++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int vec = 16 * v + 4 * g + j;
-#pragma unroll
-                for (int r = 0; r < RT; r++) {
-                    const uint32_t row = 16u * (tw + r) + m;
-                    if (r < cnt && vec < nv && row < (uint32_t)rows)
-                        __builtin_nontemporal_store(acc[r][v][j], out + (size_t)vec * rows + row);
+                if (p + 1 < np) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    group<F, VT, 1>(it + 1, xs[1], si[1], acc);
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(1, 0, p + 3);
+                    xput(p + 2);
+                    xload(p + 3);
                 }
             }
+            sync();
+            if (const int q = p + (RT > 1 ? 1 : 2); q % kChunk == 0 && q < np) flush(q);
+        }
+        flush(np);
     }
 }
 

@@ -90,8 +90,10 @@ int gs_qmatrix_shape(const gs_qmatrix *m, uint32_t *qtype, size_t *rows, size_t 
  * cores take them together), larger B goes in groups of up to 32.  The sums
  * are f32; x is split into three f16 parts, which hold all 24 bits of every
  * value of at least 2^-16 of the largest of its 256 columns (256 k .. 256 k +
- * 255 of one vector), and a smaller one to 2^-40 of that largest.  An infinity or NaN in a vector makes its own
- * logits non-finite and no other vector's. */
+ * 255 of one vector), and a smaller one to 2^-40 of that largest.  A vector's
+ * logits are the same bits whatever B is and whatever the other vectors are;
+ * an infinity or NaN in it makes its own logits non-finite and no other
+ * vector's. */
 int gs_gemv(const gs_qmatrix *m, const float *d_x, size_t B, float *d_out, void *stream);
 
 #ifdef __cplusplus

@@ -535,6 +535,33 @@ def test_gemv_x_is_whole(gpu, torch, qt, B):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("qt", ALL_TYPES)
+@pytest.mark.parametrize("rows,cols", [
+    (1000, 3584), (40000, 768), (140000, 256),      # one to five row tiles per wave, odd and even record counts
+    (33, 4096), (300, 4352), (50, 16384),           # 16 records, 17 and 64: one chunk of them, two and four
+    (2000, 1056),                                   # (32-wide types) a record of 32 columns
+])
+def test_gemv_vector_is_its_own(gpu, torch, qt, rows, cols):
+    """A vector's logits do not depend on the other vectors of the call: B of
+    them give bit for bit what each gives alone."""
+    import workloads
+    if cols % workloads.QBLOCK[qt][0]:
+        pytest.skip("not a row of this type")
+    rng = np.random.default_rng(rows + cols + qt)
+    x = torch.from_numpy((rng.standard_normal((40, cols)) * np.exp(rng.standard_normal(cols))).astype(np.float32)).cuda()
+    m = gpu.QMatrix(qt, workloads.synth_qblocks(qt, rows, cols, seed=qt), rows, cols)
+    print("gemv alone", qt, rows, cols, flush=True)
+    alone = torch.zeros((40, rows), device="cuda")
+    for b in range(40):
+        m.gemv(x[b], alone[b], B=1)
+    for B in (2, 4, 5, 16, 17, 32, 40):
+        d_o = torch.zeros((B, rows), device="cuda")
+        m.gemv(x, d_o, B=B)
+        assert torch.equal(d_o.view(torch.int32), alone[:B].view(torch.int32)), B
+    m.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("qt,cols", [(Q4_0, 32), (Q4_0, 288), (Q4_1, 96), (Q8_0, 480), (Q8_0, 2016)])
 @pytest.mark.parametrize("B", [1, 7, 20])
 def test_gemv_ragged_columns(gpu, torch, oracle, qt, cols, B):
