@@ -131,7 +131,9 @@ constexpr f4_t kZero = {0.0f, 0.0f, 0.0f, 0.0f};
 //   kHalf  a scale for each 16 columns (a lane's first four of a step, and the
 //          other four), so a sum for each;
 //   kRecScale a factor of the whole record, rec();
-//   kMin   a term min_scale() * (min_frag() . the sums of x over 32 columns);
+//   kMin   a term min_scale() * (min_frag() . the sums of x over 32 columns),
+//          min_frag() with the factor of the sums' parts (low()) where that
+//          is exact (kMinLow);
 //   Item, load(); frag(): the operand of a step; sub(): its scale (its half's);
 //   put(): a lane's part of a record from the 256 (or 8 x 32) GGUF blocks of
 //          its row.
@@ -149,6 +151,11 @@ struct Src {
     __device__ uint32_t half(int j, int i) const { return at(j, i) | at(j, i + 1) << 8; }
 };
 
+// x's parts b and c carry this factor (below); of its sums' parts, group g of
+// an operand's lanes holds part g.
+constexpr float kLow = 2048.0f;
+__device__ __forceinline__ float low() { return (threadIdx.x & 63) < 16 ? 1.0f : 1.0f / kLow; }
+
 // Bytes 2 i, 2 i + 1 of w as integers less off.
 __device__ __forceinline__ h2_t two(uint32_t w, int i, float off)
 {
@@ -161,7 +168,7 @@ __device__ __forceinline__ h2_t two(uint32_t w, int i, float off)
 // byte l of a block's 16 holds weight l (low nibble) and l + 16 (high).
 template <bool Q41> struct Q4Fmt {
     static constexpr int kRec = 2048 + 256 + (Q41 ? 256 : 0), kBlock = Q41 ? 20 : 18, kCols = 32;
-    static constexpr bool kSplit = true, kSwap = true, kHalf = false, kRecScale = false, kMin = Q41;
+    static constexpr bool kSplit = true, kSwap = true, kHalf = false, kRecScale = false, kMin = Q41, kMinLow = false;
     struct Item { u4_t q[2], d, m; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -196,7 +203,7 @@ template <bool Q41> struct Q4Fmt {
 // Q8_0: w = q d, int8 q, stored as q + 128.
 struct Q8Fmt {
     static constexpr int kRec = 4096 + 256, kBlock = 34, kCols = 32;
-    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kRecScale = false, kMin = false;
+    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kRecScale = false, kMin = false, kMinLow = false;
     struct Item { u4_t q[4], d; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -244,7 +251,7 @@ __device__ inline uint32_t k4_min(const Src &s, int o, int j)
 // the nibbles.
 template <bool Q5> struct KFmt {
     static constexpr int kRec = 2048 + (Q5 ? 512 : 0) + 256 + 64, kBlock = Q5 ? 176 : 144, kCols = 256;
-    static constexpr bool kSplit = false, kSwap = true, kHalf = false, kRecScale = true, kMin = true;
+    static constexpr bool kSplit = false, kSwap = true, kHalf = false, kRecScale = true, kMin = true, kMinLow = true;
     struct Item { u4_t q[2]; u2_t h, sc, mn; uint32_t dd; };
     static constexpr int kH = 2048, kS = 2048 + (Q5 ? 512 : 0), kM = kS + 128, kD = kS + 256;
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
@@ -278,7 +285,8 @@ template <bool Q5> struct KFmt {
     static __device__ __forceinline__ float rec(const Item &it) { return h2f(it.dd & 0xffffu); }
     static __device__ __forceinline__ h8_t min_frag(const Item &it)
     {
-        return cat(two(it.mn[0], 0, 0.0f), two(it.mn[0], 1, 0.0f), two(it.mn[1], 0, 0.0f), two(it.mn[1], 1, 0.0f));
+        const h2_t f = splat(low());
+        return cat(two(it.mn[0], 0, 0.0f) * f, two(it.mn[0], 1, 0.0f) * f, two(it.mn[1], 0, 0.0f) * f, two(it.mn[1], 1, 0.0f) * f);
     }
     static __device__ __forceinline__ float min_scale(const Item &it) { return -64.0f * h2f(it.dd >> 16); }
     static __device__ void put(uint8_t *r, const Src &s, int lane)
@@ -316,7 +324,7 @@ template <bool Q5> struct KFmt {
 // are summed apart and scaled in f32.
 struct Q6Fmt {
     static constexpr int kRec = 2048 + 1024 + 256 + 32, kBlock = 210, kCols = 256;
-    static constexpr bool kSplit = true, kSwap = true, kHalf = true, kRecScale = true, kMin = false;
+    static constexpr bool kSplit = true, kSwap = true, kHalf = true, kRecScale = true, kMin = false, kMinLow = false;
     struct Item { u4_t q[2], c, sc; uint32_t d; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -369,7 +377,7 @@ struct Q6Fmt {
 // weights.
 struct Q3Fmt {
     static constexpr int kRec = 2048 + 256 + 32, kBlock = 110, kCols = 256;
-    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kRecScale = true, kMin = false;
+    static constexpr bool kSplit = false, kSwap = false, kHalf = false, kRecScale = true, kMin = false, kMinLow = false;
     struct Item { u4_t q[2]; u2_t sc; uint32_t d; };
     static __device__ __forceinline__ void load(Item &it, gptr r, uint32_t lane)
     {
@@ -417,12 +425,15 @@ struct Q3Fmt {
 };
 
 // ------------------------------------------------------- x in f16 parts ----
-// x s = a + b + c, three f16 parts with their 11 bits each, s = 2^(15 - e)
-// for the largest |x| in [2^e, 2^(e+1)) of the record's 256 columns of the
-// vector.  Every x of at least 2^-16 of that largest is held exactly (24
-// bits: the parts are cut off, not rounded, and c has two bits left to hold);
-// a smaller one to half of f16's last step, 2^-40 of the largest.  (kMin) the
-// sums of x s over 32 columns, over 64, go into three parts too.
+// x s = a + (b + c) 2^-11, three f16 parts with their 11 bits each, s =
+// 2^(15 - e) for the largest |x| in [2^e, 2^(e+1)) of the record's 256 columns
+// of the vector.  Every x of at least 2^-27 of that largest is held exactly
+// (24 bits: the parts are cut off, not rounded, and c has two bits left to
+// hold); a smaller one to half of f16's last step in c, 2^-51 of the largest.
+// (b and c are summed apart from a, so their factor costs nothing: without it
+// the limits were 2^-16 and 2^-40.)  (kMin) the sums of x s over 32 columns,
+// over 64, go into three parts too: whole from 2^-21 of the largest x, to
+// 2^-45 of it below.
 //
 // A wave converts a record of a vector: lane L holds columns 4 L .. 4 L + 3,
 // those of step L / 8.
@@ -442,11 +453,13 @@ __device__ __forceinline__ float rest(float t, _Float16 a) { return __builtin_am
 __device__ __forceinline__ void x_split2(float x, float y, h2_t (&q)[3])
 {
     q[0] = cut(x, y);
-    x = rest(x, q[0].x);
-    y = rest(y, q[0].y);
+    x = rest(x, q[0].x) * kLow;
+    y = rest(y, q[0].y) * kLow;
     q[1] = cut(x, y);
     q[2] = h2_t{(_Float16)(x - (float)q[1].x), (_Float16)(y - (float)q[1].y)};
 }
+// The sum of x's products, from those of a and those of b and c.
+__device__ __forceinline__ float whole(float a, float bc) { return fmaf(bc, 1.0f / kLow, a); }
 // The value of a lane paired with this one (of 2, 4, 8 or 16 lanes that hold
 // equal halves).
 template <int C> __device__ __forceinline__ float pair(float x)
@@ -602,8 +615,8 @@ __device__ __forceinline__ void x_ops(XOps &o, const f4_t (&raw)[kVecs], _Float1
         if (v < nv) put(v, F::kHalf ? ph : 1, r[v].q[1]);
     lds_fence();
     o.b = F::kHalf ? from(q >= 2, q & 1) : from(q == 1, 1);
-    if constexpr (F::kMin)      // (g = 3, other rows: zeros)
-        o.sx = *reinterpret_cast<const h8_t *>(on && q == 0 && g < 3 ? sxs + 24 * (m >> 2) + 8 * g : lds + kXZeros);
+    if constexpr (F::kMin)      // part g of the sums in row 4 v (not kMinLow: b's and c's in row 4 v + 1)
+        o.sx = *reinterpret_cast<const h8_t *>(on && g < 3 && q == (!F::kMinLow && g > 0) ? sxs + 24 * (m >> 2) + 8 * g : lds + kXZeros);
 }
 
 // A record's sum for the lane's row and vector, times s.
@@ -614,11 +627,14 @@ template <class F> __device__ __forceinline__ float dot(const typename F::Item &
     for (int ks = 0; ks < 8; ks++) {
         const h8_t w = F::frag(it, ks);
         const f4_t D = mfma(*reinterpret_cast<const h8_t *>(x.b + 32 * ks), w, mfma(x.ac[ks], w, kZero));
-        v = fmaf(D[0] + D[F::kHalf ? 2 : 1], F::sub(it, ks, 0), v);
-        if constexpr (F::kHalf) v = fmaf(D[1] + D[3], F::sub(it, ks, 1), v);
+        v = fmaf(whole(D[0], D[F::kHalf ? 2 : 1]), F::sub(it, ks, 0), v);
+        if constexpr (F::kHalf) v = fmaf(whole(D[1], D[3]), F::sub(it, ks, 1), v);
     }
     if constexpr (F::kRecScale) v *= F::rec(it);
-    if constexpr (F::kMin) v = fmaf(mfma(x.sx, F::min_frag(it), kZero)[0], F::min_scale(it), v);
+    if constexpr (F::kMin) {
+        const f4_t D = mfma(x.sx, F::min_frag(it), kZero);
+        v = fmaf(F::kMinLow ? D[0] : whole(D[0], D[1]), F::min_scale(it), v);
+    }
     return v;
 }
 
@@ -752,7 +768,7 @@ __device__ __forceinline__ void group(const typename F::Item *it, const _Float16
                                                              : h8_t{0, 0, 0, 0, f[r][4], f[r][5], f[r][6], f[r][7]};
                     const f4_t E = mfma(xb, w, mfma(xc, w, kZero)), D = mfma(xa, w, kZero);
 #pragma unroll
-                    for (int j = 0; j < 4; j++) sum[r][v][j] = fmaf(D[j] + E[j], s[r][i], sum[r][v][j]);
+                    for (int j = 0; j < 4; j++) sum[r][v][j] = fmaf(whole(D[j], E[j]), s[r][i], sum[r][v][j]);
                 }
             // these sums are done here (else the steps of a record are mixed
             // until the registers spill)
@@ -769,17 +785,26 @@ __device__ __forceinline__ void group(const typename F::Item *it, const _Float16
 #pragma unroll
     for (int v = 0; v < VT; v++) {
         const f4_t iv = *reinterpret_cast<const f4_t *>(inv + 16 * v + 4 * (lane >> 4));
-        h8_t sx;
-        if constexpr (F::kMin) sx = *reinterpret_cast<const h8_t *>(xb + VT * 3 * 8 * kXStep + 512 * v + 8 * lane);
+        h8_t sa, sb;            // the sums' parts (not kMinLow: a, and b and c)
+        if constexpr (F::kMin) {
+            constexpr h8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
+            const h8_t sx = *reinterpret_cast<const h8_t *>(xb + VT * 3 * 8 * kXStep + 512 * v + 8 * lane);
+            sa = F::kMinLow || lane < 16 ? sx : z;
+            sb = lane < 16 ? z : sx;
+        }
 #pragma unroll
         for (int r = 0; r < N; r++) {
-            f4_t D;
-            if constexpr (F::kMin) D = mfma(sx, F::min_frag(it[r]), kZero);
+            f4_t D, E;
+            if constexpr (F::kMin) {
+                const h8_t w = F::min_frag(it[r]);
+                D = mfma(sa, w, kZero);
+                if constexpr (!F::kMinLow) E = mfma(sb, w, kZero);
+            }
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 float t = sum[r][v][j];
                 if constexpr (F::kRecScale) t *= F::rec(it[r]);
-                if constexpr (F::kMin) t = fmaf(D[j], F::min_scale(it[r]), t);
+                if constexpr (F::kMin) t = fmaf(F::kMinLow ? D[j] : whole(D[j], E[j]), F::min_scale(it[r]), t);
                 acc[r][v][j] += t * iv[j];
             }
         }

@@ -89,8 +89,10 @@ int gs_qmatrix_shape(const gs_qmatrix *m, uint32_t *qtype, size_t *rows, size_t 
  * decode step; up to 32 vectors share one pass over the weights (the matrix
  * cores take them together), larger B goes in groups of up to 32.  The sums
  * are f32; x is split into three f16 parts, which hold all 24 bits of every
- * value of at least 2^-16 of the largest of its 256 columns (256 k .. 256 k +
- * 255 of one vector), and a smaller one to 2^-40 of that largest.  A vector's
+ * value of at least 2^-27 of the largest of its 256 columns (256 k .. 256 k +
+ * 255 of one vector), and a smaller one to 2^-51 of that largest; the sums of
+ * 32 values that the minimums of Q4_1, Q4_K and Q5_K multiply are held from
+ * 2^-21 of it, and to 2^-45.  A vector's
  * logits are the same bits whatever B is and whatever the other vectors are;
  * an infinity or NaN in it makes its own logits non-finite and no other
  * vector's. */

@@ -536,6 +536,64 @@ def test_gemv_x_is_whole(gpu, torch, qt, B):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("qt", ALL_TYPES)
+@pytest.mark.parametrize("B", [1, 5, 17])
+def test_gemv_x_range(gpu, torch, qt, B):
+    """With one weight of 1 per row every x of at least 2^-27 of its record's
+    largest comes back bit for bit, and a smaller one to 2^-51 of the largest."""
+    n = 512
+    rng = np.random.default_rng(100 * qt + B)
+    mant = rng.integers(1 << 23, 1 << 24, (B, n)).astype(np.float64) * rng.choice([-1.0, 1.0], (B, n))
+    x = mant * 2.0 ** (rng.integers(-26, 1, (B, n)) - 23)       # [2^-26, 2)
+    x[:, ::256] = 1.9375
+    small = x.copy()
+    small[:, 1::2] *= 2.0 ** -14
+    m = gpu.QMatrix(qt, _unit_blocks(qt, n, n, np.arange(n)), n, n)
+    d_o = torch.zeros((B, n), device="cuda")
+    print("gemv x range", qt, B, flush=True)
+    m.gemv(torch.from_numpy(x.astype(np.float32)).cuda(), d_o, B=B)
+    assert np.array_equal(_f32_bits(d_o.cpu().numpy()), _f32_bits(x.astype(np.float32)))
+    m.gemv(torch.from_numpy(small.astype(np.float32)).cuda(), d_o, B=B)
+    assert (np.abs(d_o.cpu().numpy() - small) <= 2.0 ** -50).all()
+    m.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", [Q4_1, Q4_K, Q5_K])
+@pytest.mark.parametrize("B", [1, 5, 17])
+def test_gemv_minimums_range(gpu, torch, oracle, qt, B):
+    """The minimums' sums of x: row r is 1 (or -1) at the columns of sub-block
+    r and 0 elsewhere.  A value 2^20 times the others, in a sub-block of the
+    record that these rows do not take, costs them nothing: a sum of 32 is good
+    to the roundings of its additions (a tree of five levels)."""
+    import workloads
+    w, nb = workloads.QBLOCK[qt]
+    n, rows = 512, 16
+    b = np.zeros((rows, n // w, nb), np.uint8)
+    r = np.arange(rows)
+    one = np.array([1.0], np.float16).view(np.uint8)
+    if qt == Q4_1:
+        b[r, r, 2:4] = one
+    else:
+        b[:, :, 0:2] = one
+        b[:, :, 2:4] = one
+        b[r, r // 8, 8 + r % 8] = np.where(r % 8 < 4, 1, 16)
+    want_w = np.repeat(np.eye(rows), 32, axis=1) * (1 if qt == Q4_1 else -1)
+    assert np.array_equal(oracle.dequant(qt, b.reshape(-1), rows * n).reshape(rows, n), want_w)
+    rng = np.random.default_rng(10 * qt + B)
+    x = rng.standard_normal((B, n)).astype(np.float32)
+    x[:, [5, 300]] = np.float32(1.37 * 2.0 ** 20)
+    m = gpu.QMatrix(qt, b.reshape(-1), rows, n)
+    d_o = torch.zeros((B, rows), device="cuda")
+    print("gemv minimums", qt, B, flush=True)
+    m.gemv(torch.from_numpy(x).cuda(), d_o, B=B)
+    got = d_o.cpu().numpy().astype(np.float64)
+    m.close()
+    ex, ab = x.astype(np.float64) @ want_w.T, np.abs(x.astype(np.float64)) @ np.abs(want_w).T
+    assert (np.abs(got - ex) <= 6 * 2.0 ** -24 * ab).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", ALL_TYPES)
 @pytest.mark.parametrize("rows,cols", [
     (1000, 3584), (40000, 768), (140000, 256),      # one to five row tiles per wave, odd and even record counts
     (33, 4096), (300, 4352), (50, 16384),           # 16 records, 17 and 64: one chunk of them, two and four
