@@ -107,13 +107,27 @@ __device__ __forceinline__ int f_bin(float dp)
 // that is a normal float is no midpoint of two floats and lies 2^-49 or
 // more from the next one, so rounding the product to float gives x / T
 // itself (infinities, zeros, NaN and overflow too).  A quotient below 2^-126
-// may be one of its steps (2^-149) off where it is a midpoint; no summand
-// sees that: y - m rounds to -m, or is so small that its exp is 1.
+// may be one of its steps (2^-149) off where it is a midpoint.  No summand
+// sees that (y - m rounds to -m, or is so small that its exp is 1), but the
+// order of the row does: rows with such elements are left to the sort
+// (f_may_tie).
 // Where the passes are bound by issue: 8 rows at V 50257 129.8 -> 124.9 us
 // (passes 2 and 3 18.7 + 13.2 -> 17.0 + 10.7 us), 300 rows at V 100000
 // 317 -> 300 us, 512 mixed rows at V 256000 351 -> 329 us.  256 rows at
 // V 152064 stay at 230..233 us: their passes wait for the caches (4 TB/s).
 __device__ __forceinline__ float f_scaled(float x, double iT) { return (float)((double)x * iT); }
+// May x / T be a midpoint of two floats below 2^-126, and the product lie
+// beside it?  Such an x is j T / 2 steps of 2^-149 with j odd, a whole number:
+// T is even.  With 1 / T off by a factor 1 + d the product is j (1 + d) / 2
+// steps before its rounding to double, and rounds to j / 2 if |d| <= 2^-54
+// (half an ulp of j is more than j 2^-54).  The least other T is 98.
+__device__ __forceinline__ bool f_may_tie(float T)
+{
+    return T >= 2.0f && 0.5f * T == truncf(0.5f * T) &&
+           fabs(fma((double)T, 1.0 / (double)T, -1.0)) > 0x1p-54;      // (an infinite T: NaN)
+}
+// Is x a value whose quotient f_scaled may miss (where f_may_tie(T))?
+__device__ __forceinline__ bool f_tiny(float x, float T) { return x != 0.0f && fabsf(x) < T * 0x1p-126f; }
 __device__ __forceinline__ uint64_t f_entry(float y, uint32_t i) { return ((uint64_t)f2key(y) << 32) | (uint64_t)(~i); }
 __device__ __forceinline__ float f_entry_y(uint64_t en) { return key2f((uint32_t)(en >> 32)); }
 __device__ __forceinline__ uint32_t f_entry_id(uint64_t en) { return ~(uint32_t)en; }

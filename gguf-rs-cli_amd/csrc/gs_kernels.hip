@@ -81,6 +81,9 @@ struct RowSmem {
         Full3Smem f3;
     } x;
     int clast;                                  // chunk_rows_kernel: this block finishes the row
+    // sample_row<kModeBins>: the row holds quotients that f_scaled may miss
+    // (a word before the buffers moves them all: 2% on full-vocabulary rows)
+    int flag_tied;
 };
 
 // --------------------------------------------------------------------------
@@ -1412,6 +1415,17 @@ __device__ __forceinline__ void sample_row(RowSmem &sm, const RowArgs &a, int b,
 #endif
     const float *row = crow ? a.cvrow + (size_t)b * a.cvld : a.logits + (size_t)b * a.ld;
     if (t == 0) { sm.nuniq = 0; sm.flag_nan = 0; }
+    if (MODE == kModeBins) {
+        // The binned forms scale by a product; a row whose quotients that may
+        // miss is sorted whole.  (Looked for here, where few registers are
+        // taken: next to the binned forms it cost them 2%.)
+        if (t == 0) sm.flag_tied = 0;
+        if (f_may_tie(p.temperature)) {
+            __syncthreads();
+            for (int i = t; i < V; i += kThreads)
+                if (f_tiny(ldg(row + i), p.temperature)) sm.flag_tied = 1;
+        }
+    }
 
     int tok = 0, status = GS_OK;
     const bool has_pen = !crow && (p.rep_penalty != 1.0f) && a.recent != nullptr;
@@ -1463,6 +1477,11 @@ __device__ __forceinline__ void sample_row(RowSmem &sm, const RowArgs &a, int b,
     if (regpath) reg_clear(sm, has_pen, V);   // the register path builds its penalty table itself
     __syncthreads();
     if (has_pen && !regpath) build_penalty(sm, pl, p.temperature > 0.0f ? p.temperature : 1.0f, p.rep_penalty);
+    if (MODE == kModeBins && has_pen && f_may_tie(p.temperature)) {
+        for (int i = t; i < kHashSlots; i += kThreads)
+            if (sm.hkey[i] != kEmpty && f_tiny(__uint_as_float(sm.hval[i]), p.temperature)) sm.flag_tied = 1;
+        __syncthreads();
+    }
     if (wsrc && t < W) pl.id = rid;        // tested against V by the register paths
     GS_STAMP(8 * MODE + 1);
 
@@ -1507,13 +1526,13 @@ __device__ __forceinline__ void sample_row(RowSmem &sm, const RowArgs &a, int b,
     } else if (MODE == kModeBins) {
         bool done = false;
         if (sm.flag_nan) { status = GS_ERR_NAN; done = true; }
-        else if (keep == V && ((reinterpret_cast<uintptr_t>(row) & 3u) == 0)) {
+        else if (keep == V && !sm.flag_tied && ((reinterpret_cast<uintptr_t>(row) & 3u) == 0)) {
             uint64_t *gl = reinterpret_cast<uint64_t *>(a.scratch + (size_t)b * a.scratch_stride);
             const uint32_t lcap = (uint32_t)(a.scratch_stride / 2);
             done = full_v3_row(sm, row, V, p.temperature, p.top_p, has_pen, r, gl, lcap, &tok, &status);
         }
         if (t == 0) a.fb[b] = done ? 0 : 1;
-        if (!done && keep == V && ((reinterpret_cast<uintptr_t>(row) & 3u) == 0)) {
+        if (!done && keep == V && !sm.flag_tied && ((reinterpret_cast<uintptr_t>(row) & 3u) == 0)) {
             // the first binned form (per-bin classes and thresholds)
             __syncthreads();
             uint64_t *gl = reinterpret_cast<uint64_t *>(a.scratch + (size_t)b * a.scratch_stride);
