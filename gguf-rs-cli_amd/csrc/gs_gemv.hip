@@ -523,6 +523,7 @@ template <class F> __device__ __forceinline__ void x_place(int lane, int &g, int
 constexpr int kChunk = 16;
 
 // ------------------------------------------------- up to 4 vectors (GEMV) ---
+// (and more over few rows, four to a block)
 // Rows 4 v and 4 v + 1 of the first MFMA's A = parts a and c of vector v (the
 // others zero), row 4 v + 1 of the second one's = b: a lane's sums of vector
 // g are D[0] and D[1].  Formats with a scale for each 16 columns (kHalf) use
@@ -640,13 +641,16 @@ template <class F> __device__ __forceinline__ float dot(const typename F::Item &
 
 template <class F, bool MULTI>
 __global__ void __launch_bounds__(64 * kMaxWaves)
-qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, int np, int nv, int tiles, int tpb)
+qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, int np, int B, int tiles, int tpb)
 {
     extern __shared__ __align__(16) float red[];    // [2][batch] sums of a tile, then the waves' x
     const int lane = threadIdx.x & 63, nw = blockDim.x >> 6, ts = lds_tile(nw);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t0 = blockIdx.x * tpb, t1 = min(t0 + tpb, tiles);
+    const int v0 = kVecs * blockIdx.y, nv = min(kVecs, B - v0);
     if (t0 >= t1) return;
+    x += (size_t)v0 * cols;
+    out += (size_t)v0 * rows;
     _Float16 *xl = reinterpret_cast<_Float16 *>(red + 2 * kBatch * ts) + kXWave * w;
     XOps xo;
     typename F::Item it[kInFlight];
@@ -683,8 +687,9 @@ qgemv_kernel(const uint8_t *W, const float *x, float *out, int rows, int cols, i
                     default: __builtin_amdgcn_s_setprio(0); break;
                     }
 #pragma unroll
-                    for (int d = 0; d < kInFlight; d++) {       // (a tile past nb: not used)
+                    for (int d = 0; d < kInFlight; d++) {
                         const int k = k0 + d;
+                        if (d > 0 && k >= nb) break;
                         const float v = dot<F>(it[d], xo) * xo.inv;
                         __builtin_amdgcn_sched_barrier(0);
                         load(d, tb + k + kInFlight, p);
@@ -1034,10 +1039,9 @@ int gemv(const gs_qmatrix *m, const float *x, float *out, int B, hipStream_t st)
 {
     const int nw = MULTI ? gs::kMaxWaves : m->np;
     int blocks = m->cus * (gs::kMaxWaves / nw);         // 16 waves per CU
-    int tpb = (m->tiles + blocks - 1) / blocks;
-    tpb = (tpb + gs::kInFlight - 1) / gs::kInFlight * gs::kInFlight;
+    const int tpb = (m->tiles + blocks - 1) / blocks;
     blocks = (m->tiles + tpb - 1) / tpb;
-    hipLaunchKernelGGL((gs::qgemv_kernel<F, MULTI>), dim3(blocks), dim3(64 * nw), gs::gemv_lds(nw), st, m->base, x, out,
+    hipLaunchKernelGGL((gs::qgemv_kernel<F, MULTI>), dim3(blocks, (B + gs::kVecs - 1) / gs::kVecs), dim3(64 * nw), gs::gemv_lds(nw), st, m->base, x, out,
                        (int)m->rows, (int)m->cols, m->np, B, m->tiles, tpb);
     return hipGetLastError() == hipSuccess ? GS_OK : GS_ERR_HIP;
 }
@@ -1071,7 +1075,20 @@ int gemm(const gs_qmatrix *m, const float *x, float *out, int B, int per, int gr
 template <class F>
 int project(const gs_qmatrix *m, const float *x, float *out, int B, hipStream_t st)
 {
-    if (B <= gs::kVecs)
+    // More than 4 vectors over few rows: a wave of the second kernel takes row
+    // tiles through all columns, so fewer tiles than its waves (8 per CU) leave
+    // some without work, and the time is that of one tile.  There the first
+    // kernel takes the vectors four at a time (the same bits).  The line: 6
+    // (row tile, four vectors) pairs per CU.  us per call by the second kernel
+    // and the first, on the near and far side of it:
+    //                     4000 rows: 5, 16, 24, 32 vectors         8000 rows: 8, 12, 16
+    //   Q4_K x 3584       30.8 11.8  31.0 26.6  51.2 38.3 50.8 49.8  30.8 16.3  30.8 23.7  30.7 31.1
+    //   Q6_K x 8192       79.4 33.6  78.3 71.0  131 104   132 137    85.4 50.4  85.4 74.5  83.1 93.7
+    //   Q8_0 x 3584       27.1 12.8  28.1 25.9  45.9 38.5 46.2 49.6  29.1 17.5  29.5 25.8  28.7 35.6
+    // (one vector after the other on the vector units, 4000 rows, 5 vectors:
+    // Q6_K x 8192 68, Q8_0 x 3584 26.9)
+    const bool few = (size_t)((B + gs::kVecs - 1) / gs::kVecs) * m->tiles <= 6 * (size_t)m->cus;
+    if (B <= gs::kVecs || few)
         return m->np <= gs::kMaxWaves ? gemv<F, false>(m, x, out, B, st) : gemv<F, true>(m, x, out, B, st);
     const int groups = (B + 31) / 32, per = (B + groups - 1) / groups;
     return per <= 16 ? gemm<F, 1>(m, x, out, B, per, groups, st) : gemm<F, 2>(m, x, out, B, per, groups, st);

@@ -620,6 +620,37 @@ def test_gemv_vector_is_its_own(gpu, torch, qt, rows, cols):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("qt", ALL_TYPES)
+@pytest.mark.parametrize("rows,cols,Bs", [
+    (3072, 4352, (31, 32, 33, 40)),     # 192 row tiles, 17 records: eight groups of four vectors, and nine
+    (12288, 768, (5, 8, 9)),            # 768 row tiles: two groups, and three
+    (12289, 1280, (5, 8)),              # one row more
+    (13000, 1056, (5, 20)),             # (32-wide types) a record of 32 columns
+    (3300, 16384, (29, 32)),            # 64 records
+])
+def test_gemv_few_rows(gpu, torch, qt, rows, cols, Bs):
+    """Both sides of the line between the two kernels for more than 4 vectors
+    (6 pairs of a row tile and four vectors per CU, 256 CUs): every vector's
+    logits are those it gives alone, bit for bit."""
+    import workloads
+    if cols % workloads.QBLOCK[qt][0]:
+        pytest.skip("not a row of this type")
+    rng = np.random.default_rng(rows + cols + qt)
+    n = max(Bs)
+    x = torch.from_numpy((rng.standard_normal((n, cols)) * np.exp(rng.standard_normal(cols))).astype(np.float32)).cuda()
+    m = gpu.QMatrix(qt, workloads.synth_qblocks(qt, rows, cols, seed=qt), rows, cols)
+    print("gemv few rows", qt, rows, cols, flush=True)
+    alone = torch.zeros((n, rows), device="cuda")
+    for b in range(n):
+        m.gemv(x[b], alone[b], B=1)
+    for B in Bs:
+        d_o = torch.zeros((B, rows), device="cuda")
+        m.gemv(x, d_o, B=B)
+        assert torch.equal(d_o.view(torch.int32), alone[:B].view(torch.int32)), B
+    m.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("qt,cols", [(Q4_0, 32), (Q4_0, 288), (Q4_1, 96), (Q8_0, 480), (Q8_0, 2016)])
 @pytest.mark.parametrize("B", [1, 7, 20])
 def test_gemv_ragged_columns(gpu, torch, oracle, qt, cols, B):
