@@ -619,6 +619,61 @@ def test_gemv_vector_is_its_own(gpu, torch, qt, rows, cols):
     m.close()
 
 
+# Error of a vector's logits against 64-bit sums, 2-norm over 2-norm, x normal.
+# A result goes through some 30 roundings (8 steps of a record, its minimums,
+# up to 16 records, the chunks), each of 0.29 2^-23 rms of a running sum that
+# grows to the result: about 1.3e-7 (measured: up to 1.7e-7).  The bound is
+# three times that, and for one logit 2^-18 of their rms.
+REL2, RELMAX = 2.0 ** -21, 2.0 ** -18
+
+
+def _rel(got, ex):
+    rms = np.sqrt(np.mean(ex * ex))
+    err = np.abs(got.astype(np.float64) - ex)
+    return np.sqrt(np.mean(err * err)) / rms, err.max() / rms
+
+
+@pytest.mark.parametrize("qt", ALL_TYPES)
+def test_gemv_error_bound_sees_the_parts(oracle, qt):
+    """With x cut to its first part (11 bits) the error is beyond both bounds,
+    a hundred times and more, for every type."""
+    import workloads
+    rows, cols = 64, 1024
+    blocks = workloads.synth_qblocks(qt, rows, cols, seed=qt)
+    x = np.random.default_rng(qt).standard_normal(cols).astype(np.float32)
+    cut = (x.view(np.uint32) & np.uint32(0xffffe000)).view(np.float32)
+    ex, _ = oracle.matvec(qt, blocks, rows, cols, x, nthreads=4, exact=True)
+    hi, _ = oracle.matvec(qt, blocks, rows, cols, cut, nthreads=4, exact=True)
+    rel, most = _rel(hi, ex)
+    assert rel > 100 * REL2 and most > 100 * RELMAX
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", ALL_TYPES)
+@pytest.mark.parametrize("rows,cols,Bs", [
+    (1000, 3584, (1, 4, 16)), (500, 8192, (1, 4, 16)),          # the kernel for up to 4 vectors
+    (12304, 1024, (5, 16, 17, 32)), (3200, 8192, (32,)),        # the kernel for more
+])
+def test_gemv_error(gpu, torch, oracle, qt, rows, cols, Bs):
+    import workloads
+    rng = np.random.default_rng(rows + cols + qt)
+    gain = np.exp(0.5 * rng.standard_normal(cols))
+    x = (rng.standard_normal((max(Bs), cols)) * gain).astype(np.float32)
+    blocks = workloads.synth_qblocks(qt, rows, cols, seed=rows + qt)
+    m = gpu.QMatrix(qt, blocks, rows, cols)
+    worst = (0.0, 0.0)
+    for B in Bs:
+        d_o = torch.zeros((B, rows), device="cuda")
+        m.gemv(torch.from_numpy(x).cuda(), d_o, B=B)
+        got = d_o.cpu().numpy()
+        for b in {0, B - 1}:
+            ex, _ = oracle.matvec(qt, blocks, rows, cols, x[b], nthreads=8, exact=True)
+            worst = tuple(map(max, worst, _rel(got[b], ex)))
+    m.close()
+    print("gemv error", qt, rows, cols, "%.2e %.2e" % worst, flush=True)
+    assert worst[0] <= REL2 and worst[1] <= RELMAX
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("qt", ALL_TYPES)
 @pytest.mark.parametrize("rows,cols,Bs", [
