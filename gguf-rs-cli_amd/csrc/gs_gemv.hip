@@ -16,21 +16,23 @@
 // instructions per weight, as long as the read itself, for one vector, and a
 // pass over the weights for each further one.  Measured (MI355X, us per call;
 // before: one pass of the vector units per vector):
-//   Q4_K 152064 x 3584:  1 vector 62 -> 57 (5.5 TB/s), 16: 980 -> 93,
-//                        32: 1970 -> 145
-//   Q6_K 152064 x 3584:  1 vector 72 -> 77 (5.8 TB/s), 16: 1160 -> 144,
-//                        32: 2330 -> 231
-//   Q5_K 32000 x 8192:   1 vector 120 -> 40
-//   Q8_0 32000 x 4096:   4 vectors 95 -> 25
+//   Q4_K 152064 x 3584:  1 vector 61 -> 54 (5.7 TB/s), 16: 980 -> 93,
+//                        32: 1975 -> 151
+//   Q6_K 152064 x 3584:  1 vector 70 -> 72 (6.2 TB/s), 16: 1157 -> 148,
+//                        32: 2330 -> 235
+//   Q5_K 152064 x 3584:  1 vector 70 -> 71; 32000 x 8192: 121 -> 38
+//   Q8_0 32000 x 4096:   4 vectors 96 -> 26
 // With x in two parts (23 bits at best) instead of three and their products
-// in one sum: 51, 78 and 115 us for Q4_K, 72, 108 and 160 for Q6_K.
+// in one sum: 50, 78 and 116 us for Q4_K, 70, 109 and 162 for Q6_K, 64 for
+// Q5_K.
 //
 // Error against 64-bit sums (2-norm, relative; x normal, channels of unequal
-// size; 1024, 3584 and 8192 columns, 1 to 32 vectors), before -> now:
-//   Q4_0 2.2-2.5e-7 -> 0.7-1.0e-7     Q4_K 1.3-1.5e-7 -> 0.9-1.2e-7
-//   Q4_1 1.8-2.1e-7 -> 1.3-1.7e-7     Q5_K 1.2-1.5e-7 -> 0.8-1.2e-7
-//   Q8_0 2.0-2.2e-7 -> 0.8-1.1e-7     Q6_K 2.0-2.2e-7 -> 0.9-1.2e-7
-//   Q3_K 1.8-2.0e-7 -> 0.8-1.1e-7
+// size; 1024 to 8192 columns, 1 to 32 vectors, means of 4 to 8 runs), before
+// -> now:
+//   Q4_0 2.0-2.3e-7 -> 0.7-1.0e-7     Q4_K 1.4-1.5e-7 -> 0.9-1.3e-7
+//   Q4_1 1.3-1.8e-7 -> 1.3e-7         Q5_K 1.3-1.5e-7 -> 0.9-1.3e-7
+//   Q8_0 1.7-2.4e-7 -> 0.8-1.1e-7     Q6_K 2.1-2.2e-7 -> 0.9-1.2e-7
+//   Q3_K 1.9-2.0e-7 -> 0.8-1.1e-7
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>
@@ -539,8 +541,9 @@ constexpr int kChunk = 16;
 // priority falls with its progress, so that the waves of a SIMD arrive
 // together (with equal priorities the youngest came late and ran the end of
 // each batch alone: Q4_K 152064 x 3584 59 us against 52, Q6_K 84 against 74).
-// Bound: the read of the weights (5.4-6.7 TB/s at 152064 x 3584).  Four tiles
-// in flight instead of two: 57 us against 52 (Q4_K).  Rows of more columns
+// Bound: the read of the weights (5.1-6.5 TB/s at 152064 x 3584; Q3_K and Q5_K,
+// the slowest, by the unpacking).  Four tiles in flight instead of two: 57 us
+// against 52 (Q4_K; these figures with x in two parts).  Rows of more columns
 // than the waves hold (MULTI) go in chunks: a batch's tiles take one chunk
 // after the other, and the running sums stay with the waves that add them.
 constexpr int kVecs = 4, kBatch = 8, kMaxWaves = kChunk, kInFlight = 2;
@@ -1151,8 +1154,8 @@ int gs_qmatrix_shape(const gs_qmatrix *m, uint32_t *qtype, size_t *rows, size_t 
 int gs_gemv(const gs_qmatrix *m, const float *d_x, size_t B, float *d_out, void *stream)
 {
     if (!m || (B > 0 && (!d_x || !d_out))) return GS_ERR_INVALID;
-    if (((uintptr_t)d_x & 15u) != 0 || (B > 1 && (m->cols & 3) != 0)) return GS_ERR_INVALID;   // x is read as float4
-    // up to 16384 vectors per launch (groups of 16 along the grid's y)
+    if (((uintptr_t)d_x & 15u) != 0) return GS_ERR_INVALID;     // x is read as float4 (columns: a multiple of 32)
+    // up to 16384 vectors per launch (groups of 4, or of up to 32, along the grid's y)
     for (size_t b = 0; b < B; b += 16384) {
         const int n = (int)(B - b < 16384 ? B - b : 16384);
         const int rc = with_format(m->qtype, [&](auto f) {

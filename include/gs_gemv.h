@@ -73,8 +73,9 @@ typedef struct gs_qmatrix gs_qmatrix;
  * The blocks are copied to the current HIP device, through a staging buffer of
  * up to 64 MB, and rearranged there (records of 16 rows x 256 columns in the
  * order the kernels read them; rows of the matrix are padded to 16 and columns
- * to 256); synchronous.  cols must be a multiple
- * of the block size (32 / 256) -- where the reference's upload returns None
+ * to 256, in memory and in what a call reads: of the 32-wide types 1056 columns
+ * take as much as 1280, and 32 as much as 256); synchronous.  cols must be a
+ * multiple of the block size (32 / 256) -- where the reference's upload returns None
  * and falls back to the CPU, this returns GS_ERR_UNSUPPORTED (for Q4_0 and Q4_1
  * the reference has no such check and would read misaligned blocks) -- and at
  * most 16384.  Other block types return GS_ERR_UNSUPPORTED, as the
@@ -87,7 +88,8 @@ int gs_qmatrix_shape(const gs_qmatrix *m, uint32_t *qtype, size_t *rows, size_t 
  * d_out[b*rows + r] = sum_c W[r][c] * d_x[b*cols + c].  Device pointers;
  * asynchronous on `stream` (NULL = default stream).  B = 1 is the reference's
  * decode step; up to 32 vectors share one pass over the weights (the matrix
- * cores take them together), larger B goes in groups of up to 32.  The sums
+ * cores take them together), larger B goes in groups of up to 32 (of 4 where
+ * rows are few).  The sums
  * are f32; x is split into three f16 parts, which hold all 24 bits of every
  * value of at least 2^-27 of the largest of its 256 columns (256 k .. 256 k +
  * 255 of one vector), and a smaller one to 2^-51 of that largest; the sums of
